@@ -468,6 +468,12 @@ int32_t launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
 
 }  // namespace
 
+bool gemm_bf16_rows_ok(int64_t M, int64_t batch);
+int32_t gemm_bf16_rows_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
+                              const void* w, int64_t ldw, const void* bias, const void* bias2, void* y,
+                              int64_t ldy, int64_t batch, int64_t sX, int64_t sW, int64_t sC,
+                              hipStream_t s);
+
 // Fast-path predicate shared with the dispatcher in gemm.hip.
 bool gemm_bf16_nt_fast_ok(int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
                           const void* w, int64_t ldw, const void* y, int64_t ldy) {
@@ -482,6 +488,8 @@ int32_t gemm_bf16_nt_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const 
                             int64_t ldx, const void* w, int64_t ldw, const void* bias,
                             const void* bias2, void* y, int64_t ldy, int64_t batch,
                             int64_t sA, int64_t sB, int64_t sC, hipStream_t s) {
+  if (gemm_bf16_rows_ok(M, batch))
+    return gemm_bf16_rows_launch(epi, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, batch, sA, sB, sC, s);
   auto A = static_cast<const uint16_t*>(x);
   auto B = static_cast<const uint16_t*>(w);
   auto b1 = static_cast<const uint16_t*>(bias);
