@@ -34,6 +34,11 @@ SIGNATURES: dict[str, tuple] = {
         _i32,
         [_i32, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i32, _p, _i64, _p],
     ),
+    "catopt_hip_linear_workspace_bytes": (_i64, [_i32, _i64, _i64, _i64, _i32]),
+    "catopt_hip_linear_ws": (
+        _i32,
+        [_i32, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i32, _p, _i64, _p, _i64, _p],
+    ),
     "catopt_hip_matmul": (
         _i32,
         [_i32, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i32, _p, _i64, _i64, _i32, _p, _i64, _i64, _p],

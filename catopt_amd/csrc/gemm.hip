@@ -1,7 +1,7 @@
 // GEMM entry points: catopt_hip_linear and catopt_hip_matmul.
 //
-// bf16 with K-contiguous, 16-byte aligned operands goes to the 256x256
-// bf16 MFMA kernel (gemm_bf16.hip).  Everything else — fp32 (the weight
+// bf16 with K-contiguous, 16-byte aligned operands goes to the bf16 MFMA
+// kernels (gemm_bf16.hip, gemm_bf16_mid.hip, gemm_bf16_skinny.hip by size).  Everything else — fp32 (the weight
 // chain of the linear-bias association form and its construction-time
 // fold), transposed operands, unaligned views — runs here on a 64x64-tile
 // kernel using the 32x32x2 fp32 MFMA, with operands staged through LDS in
@@ -9,15 +9,9 @@
 // widened to fp32 in LDS (the products are exact), so both paths
 // accumulate in fp32.
 #include "common.hpp"
+#include "gemm_bf16.hpp"
 
 namespace catopt {
-bool gemm_bf16_nt_fast_ok(int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
-                          const void* w, int64_t ldw, const void* y, int64_t ldy);
-int32_t gemm_bf16_nt_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const void* x,
-                            int64_t ldx, const void* w, int64_t ldw, const void* bias,
-                            const void* bias2, void* y, int64_t ldy, int64_t batch,
-                            int64_t strideA, int64_t strideB, int64_t strideC, hipStream_t s);
-
 namespace {
 
 constexpr int TM = 64, TN = 64, TK = 32, NTH = 256;
@@ -251,10 +245,22 @@ int32_t dispatch_paired(int32_t epi, const void* A, int64_t lda, const void* B, 
 
 using namespace catopt;
 
-extern "C" int32_t catopt_hip_linear(int32_t dtype, int64_t M, int64_t N, int64_t K,
-                                     const void* x, int64_t ldx, const void* w, int64_t ldw,
-                                     const void* bias, const void* bias2, int32_t epilogue,
-                                     void* y, int64_t ldy, void* stream) {
+extern "C" int64_t catopt_hip_linear_workspace_bytes(int32_t dtype, int64_t M, int64_t N, int64_t K,
+                                                     int32_t epilogue) {
+  if (M < 0 || N < 0 || K < 0 || epilogue < CATOPT_EPI_NONE || epilogue > CATOPT_EPI_GLU) return -1;
+  if (dtype != CATOPT_BF16 || M == 0 || N == 0 || K == 0) return 0;
+  if (M > 0x7fffffffLL || N > 0x3fffffffLL || K > 0x7fffffffLL) return 0;
+  int n_cu = 0;
+  if (gemm_cu_count(&n_cu) != CATOPT_OK) return 0;  // no device: nothing will be launched
+  const bool paired = epilogue == CATOPT_EPI_SILU_MUL || epilogue == CATOPT_EPI_GLU;
+  return gemm_bf16_mid_workspace(gemm_bf16_mid_plan(M, N, K, paired, n_cu, true), M, N, paired);
+}
+
+extern "C" int32_t catopt_hip_linear_ws(int32_t dtype, int64_t M, int64_t N, int64_t K,
+                                        const void* x, int64_t ldx, const void* w, int64_t ldw,
+                                        const void* bias, const void* bias2, int32_t epilogue,
+                                        void* y, int64_t ldy, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
   if (M < 0 || N < 0 || K < 0) return CATOPT_E_INVAL;
   if (epilogue < CATOPT_EPI_NONE || epilogue > CATOPT_EPI_GLU) return CATOPT_E_INVAL;
   if (dtype != CATOPT_F32 && dtype != CATOPT_BF16) return CATOPT_E_UNSUPPORTED;
@@ -267,7 +273,8 @@ extern "C" int32_t catopt_hip_linear(int32_t dtype, int64_t M, int64_t N, int64_
   if (M > 0x7fffffffLL || N > 0x3fffffffLL || K > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == CATOPT_BF16 && gemm_bf16_nt_fast_ok(M, N, K, x, ldx, w, ldw, y, ldy))
-    return gemm_bf16_nt_launch(epilogue, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, 1, 0, 0, 0, s);
+    return gemm_bf16_nt_launch(epilogue, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, 1, 0, 0, 0, workspace,
+                               workspace_bytes, s);
   if (dtype == CATOPT_F32 && !paired && skinny_ok(M, N, K, x, ldx, w, ldw))
     return launch_skinny(epilogue, static_cast<const float*>(x), ldx, static_cast<const float*>(w), ldw,
                          static_cast<const float*>(bias), static_cast<const float*>(bias2),
@@ -279,6 +286,13 @@ extern "C" int32_t catopt_hip_linear(int32_t dtype, int64_t M, int64_t N, int64_
   return dtype == CATOPT_BF16
              ? dispatch_epi<uint16_t, false, true>(epilogue, x, ldx, 0, w, ldw, 0, bias, bias2, y, ldy, 0, 1, M, N, K, s)
              : dispatch_epi<float, false, true>(epilogue, x, ldx, 0, w, ldw, 0, bias, bias2, y, ldy, 0, 1, M, N, K, s);
+}
+
+extern "C" int32_t catopt_hip_linear(int32_t dtype, int64_t M, int64_t N, int64_t K,
+                                     const void* x, int64_t ldx, const void* w, int64_t ldw,
+                                     const void* bias, const void* bias2, int32_t epilogue,
+                                     void* y, int64_t ldy, void* stream) {
+  return catopt_hip_linear_ws(dtype, M, N, K, x, ldx, w, ldw, bias, bias2, epilogue, y, ldy, nullptr, 0, stream);
 }
 
 extern "C" int32_t catopt_hip_matmul(int32_t dtype, int64_t batch, int64_t M, int64_t N,
@@ -298,7 +312,7 @@ extern "C" int32_t catopt_hip_matmul(int32_t dtype, int64_t batch, int64_t M, in
   if (dtype == CATOPT_BF16 && !transA && transB && strides_ok &&
       gemm_bf16_nt_fast_ok(M, N, K, A, lda, B, ldb, C, ldc))
     return gemm_bf16_nt_launch(CATOPT_EPI_NONE, M, N, K, A, lda, B, ldb, nullptr, nullptr, C, ldc,
-                               batch, strideA, strideB, strideC, s);
+                               batch, strideA, strideB, strideC, nullptr, 0, s);
 #define CATOPT_MM(T)                                                                                          \
   if (!transA && !transB) return dispatch_epi<T, false, false>(0, A, lda, strideA, B, ldb, strideB, nullptr, nullptr, C, ldc, strideC, batch, M, N, K, s); \
   if (!transA && transB) return dispatch_epi<T, false, true>(0, A, lda, strideA, B, ldb, strideB, nullptr, nullptr, C, ldc, strideC, batch, M, N, K, s);   \

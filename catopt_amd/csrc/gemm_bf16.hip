@@ -60,13 +60,13 @@
 // of logical tiles (grouped 8 M-tiles at a time), which march through K
 // together and share that XCD's L2.
 #include "common.hpp"
+#include "gemm_bf16.hpp"
 
 namespace catopt {
 namespace {
 
 constexpr int BM = 256, BN = 256, BK = 64;     // tile; K per stage (two MFMA steps of 32)
 constexpr int NT = 512;                        // 8 waves
-constexpr int ROW_BYTES = BK * 2;              // 128: one cache line per tile row per stage
 constexpr int SLOT_ROWS = 128;                 // an LDS slot: 128 rows of one stage
 constexpr int SLOT_BYTES = SLOT_ROWS * ROW_BYTES;  // 16 KB
 // LDS slots: X rows 0-127 in a ring of 3 (read by waves 0-3), X rows
@@ -80,41 +80,6 @@ constexpr int DMA_PER_PHASE = 4;               // 1 KB loads per wave per comput
 constexpr int FM = 8, FN = 4;                  // 16x16 blocks per wave along m, n
 static_assert(BN == BM && LDS_BYTES <= 160 * 1024, "geometry");
 static_assert(SLOT_BYTES / 1024 == 4 * DMA_PER_PHASE, "a group's 4 waves fill one slot per phase");
-
-// Byte offset of (row, 16-byte chunk) in a slot.
-__device__ __forceinline__ constexpr int swz(int row, int chunk) {
-  return row * ROW_BYTES + ((chunk ^ ((row >> 1) & 7)) << 4);
-}
-
-// s_waitcnt with lgkmcnt(0) and vmcnt <= n (gfx9 encoding; expcnt not waited on).
-template <int n>
-__device__ __forceinline__ void wait_vm_lgkm0() {
-  static_assert(n >= 0 && n < 64, "vmcnt field");
-  __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | ((n >> 4) << 14));
-}
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (3 << 14)); }
-
-__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-struct TileMap {
-  int tm, tn;
-};
-
-// Logical tile -> (M-tile, N-tile): groups of 8 M-tiles, N-tiles in order.
-__device__ __forceinline__ TileMap tile_of(int lt, int tiles_m, int tiles_n) {
-  constexpr int GM = 8;
-  const int per_group = GM * tiles_n;
-  const int group = lt / per_group;
-  const int first_m = group * GM;
-  const int gsize = min(tiles_m - first_m, GM);
-  const int in_group = lt - group * per_group;
-  TileMap t;
-  t.tm = first_m + in_group % gsize;
-  t.tn = in_group / gsize;
-  return t;
-}
 
 // The kernel's operands, shared by its helpers.
 struct GemmArgs {
@@ -300,73 +265,11 @@ __global__ __launch_bounds__(NT, 1) void gemm_bf16_nt(
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // ---- epilogue of the tile at (m0, n0).  acc[i][j][r] is C[m][n] with
-  // m = m0 + 128 grp + 16 j + l % 16 and n = (first column of block i) +
-  // 4 (l / 16) + r.  Adjacent blocks i, i+1 trade halves between lane rows
-  // (v_permlane16_swap) so each lane holds 8 consecutive columns: one
-  // 16-byte store per lane, 64 contiguous bytes per output row (8-byte stores
-  // of 32-byte row pieces cost 2-7% more kernel time).
+  // ---- epilogue of the tile at (m0, n0): the wave's 128 rows and 64 columns
+  // (paired: 32 of each projection)
   auto epilogue = [&](int m0, int n0) {
-    const int mrow = m0 + 128 * grp + (lane & 15);
-    const int q = lane >> 4;
-    constexpr int NBLK = PAIRED ? FN / 2 : FN;
-#pragma unroll
-    for (int i = 0; i < NBLK; i += 2) {
-      // blocks i, i+1: 4 columns per lane each -> 8 consecutive per lane
-      const int nb = PAIRED ? n0 + wq * 32 + i * 16 : n0 + wq * 64 + i * 16;
-      float bv[2][4], bv2[2][4];
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int n = nb + 16 * h + 4 * q + r;
-          bv[h][r] = (EPI == CATOPT_EPI_BIAS || EPI == CATOPT_EPI_BIAS_ADD2) && n < N ? bf16_to_f32(bias[n]) : 0.f;
-          bv2[h][r] = (EPI == CATOPT_EPI_BIAS_ADD2) && n < N ? bf16_to_f32(bias2[n]) : 0.f;
-        }
-#pragma unroll
-      for (int j = 0; j < FM; ++j) {
-        uint32_t pk[2][2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          float o[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float a = acc[i + h][j][r];
-            if (PAIRED) {
-              const float b = acc[i + h + 2][j][r];
-              o[r] = (EPI == CATOPT_EPI_SILU_MUL) ? a * __builtin_amdgcn_rcpf(1.0f + __expf(-a)) * b
-                                                  : a * __builtin_amdgcn_rcpf(1.0f + __expf(-b));
-            } else if (EPI == CATOPT_EPI_BIAS_ADD2) {
-              o[r] = (a + bv[h][r]) + bv2[h][r];
-            } else {
-              o[r] = a + bv[h][r];
-            }
-          }
-          pk[h][0] = pack_bf16x2(o[0], o[1]);
-          pk[h][1] = pack_bf16x2(o[2], o[3]);
-        }
-        // rows q = 1, 3 take block i+1 columns 0-3 / 8-11 of rows 0, 2 and
-        // give them their block i columns 4-7 / 12-15
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          auto sw = __builtin_amdgcn_permlane16_swap(pk[0][w], pk[1][w], false, false);
-          pk[0][w] = sw[0];
-          pk[1][w] = sw[1];
-        }
-        const int m = mrow + 16 * j;
-        const int n = nb + 16 * (q & 1) + 8 * (q >> 1);
-        if (m >= M || n >= N) continue;
-        uint16_t* dst = C + (int64_t)m * ldc + n;
-        if (vec_store && n + 7 < N) {
-          *reinterpret_cast<u32x4*>(dst) = u32x4{pk[0][0], pk[0][1], pk[1][0], pk[1][1]};
-        } else {
-          const uint32_t wv[4] = {pk[0][0], pk[0][1], pk[1][0], pk[1][1]};
-#pragma unroll
-          for (int r = 0; r < 8; ++r)
-            if (n + r < N) dst[r] = (uint16_t)(wv[r >> 1] >> (16 * (r & 1)));
-        }
-      }
-    }
+    gemm_epilogue<EPI, FM>(acc, m0 + 128 * grp + (lane & 15), n0 + wq * (PAIRED ? 32 : 64), M, N, bias, bias2, C,
+                           ldc, vec_store);
   };
 
   // ---- prologue: stage 0 (each wave its W and X rows) and X of stage 1
@@ -442,20 +345,10 @@ int32_t launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
   const int tiles_n = (N + (PAIRED ? BN / 2 : BN) - 1) / (PAIRED ? BN / 2 : BN);
   const int64_t nblocks = (int64_t)tiles_m * tiles_n;
   if (nblocks > 0x7fffffff || batch > 65535) return CATOPT_E_UNSUPPORTED;
-  // persistent: one workgroup per CU (each walks its tiles in rounds); the
-  // CU count is read once per device (idempotent; a race writes the same value)
-  static int cu_count[64] = {};
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return set_hip_error(e);
-  int n_cu = dev >= 0 && dev < 64 ? cu_count[dev] : 0;
-  if (n_cu == 0) {
-    int v = 0;
-    e = hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) return set_hip_error(e);
-    n_cu = v > 0 ? v : 1;
-    if (dev >= 0 && dev < 64) cu_count[dev] = n_cu;
-  }
+  // persistent: one workgroup per CU (each walks its tiles in rounds)
+  int n_cu = 0;
+  const int32_t st = gemm_cu_count(&n_cu);
+  if (st != CATOPT_OK) return st;
   const int64_t grid = nblocks < n_cu ? nblocks : n_cu;
   // the epilogue's 16-byte stores of eight columns need every row of every
   // batch of C 16-byte aligned; otherwise it stores columns one by one
@@ -468,11 +361,23 @@ int32_t launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
 
 }  // namespace
 
-bool gemm_bf16_rows_ok(int64_t M, int64_t batch);
-int32_t gemm_bf16_rows_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
-                              const void* w, int64_t ldw, const void* bias, const void* bias2, void* y,
-                              int64_t ldy, int64_t batch, int64_t sX, int64_t sW, int64_t sC,
-                              hipStream_t s);
+// The current device's CU count, read once per device (idempotent; a race
+// writes the same value).
+int32_t gemm_cu_count(int* out) {
+  static int cu_count[64] = {};
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return set_hip_error(e);
+  int n = dev >= 0 && dev < 64 ? cu_count[dev] : 0;
+  if (n == 0) {
+    e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return set_hip_error(e);
+    if (n <= 0) n = 1;
+    if (dev >= 0 && dev < 64) cu_count[dev] = n;
+  }
+  *out = n;
+  return CATOPT_OK;
+}
 
 // Fast-path predicate shared with the dispatcher in gemm.hip.
 bool gemm_bf16_nt_fast_ok(int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
@@ -487,9 +392,22 @@ bool gemm_bf16_nt_fast_ok(int64_t M, int64_t N, int64_t K, const void* x, int64_
 int32_t gemm_bf16_nt_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const void* x,
                             int64_t ldx, const void* w, int64_t ldw, const void* bias,
                             const void* bias2, void* y, int64_t ldy, int64_t batch,
-                            int64_t sA, int64_t sB, int64_t sC, hipStream_t s) {
-  if (gemm_bf16_rows_ok(M, batch))
+                            int64_t sA, int64_t sB, int64_t sC, void* ws, int64_t ws_bytes, hipStream_t s) {
+  const bool paired = epi == CATOPT_EPI_SILU_MUL || epi == CATOPT_EPI_GLU;
+  if (batch == 1) {
+    int n_cu = 0;
+    const int32_t st = gemm_cu_count(&n_cu);
+    if (st != CATOPT_OK) return st;
+    GemmMidPlan plan = gemm_bf16_mid_plan(M, N, K, paired, n_cu, ws != nullptr && aligned16(ws));
+    if (gemm_bf16_mid_workspace(plan, M, N, paired) > ws_bytes)
+      plan = gemm_bf16_mid_plan(M, N, K, paired, n_cu, false);
+    if (plan.shape == GEMM_ROWS)
+      return gemm_bf16_rows_launch(epi, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, 1, 0, 0, 0, s);
+    if (plan.shape != GEMM_MID_NONE)
+      return gemm_bf16_mid_launch(plan, epi, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, ws, s);
+  } else if (M <= 64) {
     return gemm_bf16_rows_launch(epi, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, batch, sA, sB, sC, s);
+  }
   auto A = static_cast<const uint16_t*>(x);
   auto B = static_cast<const uint16_t*>(w);
   auto b1 = static_cast<const uint16_t*>(bias);

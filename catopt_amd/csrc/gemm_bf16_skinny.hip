@@ -23,6 +23,7 @@
 // W rows feed the MFMA's A operand, so accumulator register r of lane l is
 // C[16 mb + l % 16][n0 + 4 (l / 16) + r].
 #include "common.hpp"
+#include "gemm_bf16.hpp"
 
 namespace catopt {
 namespace {
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(64 * rows_waves(MB)) void gemm_bf16_rows(
         for (int p = 0; p < NP; ++p)
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb)
-            acc[p][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][h][p], xf[u][h][mb], acc[p][mb], 0, 0, 0);
+            acc[p][mb] = mfma16(wf[u][h][p], xf[u][h][mb], acc[p][mb]);
   }
 #pragma unroll
   for (int p = 0; p < NP; ++p)
@@ -125,19 +126,10 @@ __global__ __launch_bounds__(64 * rows_waves(MB)) void gemm_bf16_rows(
   float o[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const float a = s[0][r];
     const int nn = min(n + r, N - 1);
-    if constexpr (EPI == CATOPT_EPI_SILU_MUL) {
-      o[r] = a * __builtin_amdgcn_rcpf(1.0f + __expf(-a)) * s[NP - 1][r];
-    } else if constexpr (EPI == CATOPT_EPI_GLU) {
-      o[r] = a * __builtin_amdgcn_rcpf(1.0f + __expf(-s[NP - 1][r]));
-    } else if constexpr (EPI == CATOPT_EPI_BIAS_ADD2) {
-      o[r] = (a + bf16_to_f32(bias[nn])) + bf16_to_f32(bias2[nn]);
-    } else if constexpr (EPI == CATOPT_EPI_BIAS) {
-      o[r] = a + bf16_to_f32(bias[nn]);
-    } else {
-      o[r] = a;
-    }
+    const float b1 = EPI == CATOPT_EPI_BIAS || EPI == CATOPT_EPI_BIAS_ADD2 ? bf16_to_f32(bias[nn]) : 0.f;
+    const float b2 = EPI == CATOPT_EPI_BIAS_ADD2 ? bf16_to_f32(bias2[nn]) : 0.f;
+    o[r] = epilogue_value<EPI>(s[0][r], s[NP - 1][r], b1, b2);
   }
   uint16_t* dst = C + (int64_t)m * ldc + n;
   if (vec_store && n + 3 < N) {
@@ -153,6 +145,7 @@ template <int EPI>
 int32_t launch_rows(const uint16_t* X, int64_t ldx, const uint16_t* W, int64_t ldw, const uint16_t* bias,
                     const uint16_t* bias2, uint16_t* C, int64_t ldc, int M, int N, int K, int64_t batch,
                     int64_t sX, int64_t sW, int64_t sC, hipStream_t s) {
+  if (batch > 65535) return CATOPT_E_UNSUPPORTED;
   const dim3 grid((uint32_t)((N + SKN - 1) / SKN), (uint32_t)batch), block(64 * rows_waves((M + 15) / 16));
   const int vec_store = ldc % 4 == 0 && sC % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 7) == 0;
 #define CATOPT_ROWS(MB)                                                                                    \
@@ -171,8 +164,6 @@ int32_t launch_rows(const uint16_t* X, int64_t ldx, const uint16_t* W, int64_t l
 }
 
 }  // namespace
-
-bool gemm_bf16_rows_ok(int64_t M, int64_t batch) { return M <= 64 && batch <= 65535; }
 
 int32_t gemm_bf16_rows_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
                               const void* w, int64_t ldw, const void* bias, const void* bias2, void* y,

@@ -155,8 +155,14 @@ def linear(
         if paired:
             raise NotImplementedError("paired epilogue over an empty contraction")
         return y
-    st = lib.catopt_hip_linear(dt, M, N, K, _ptr(x2), ldx, _ptr(weight), weight.stride(0),
-                               _ptr(bias), _ptr(bias2), int(epilogue), _ptr(y), N, _stream(x))
+    wsb = lib.catopt_hip_linear_workspace_bytes(dt, M, N, K, int(epilogue)) if dt == L.BF16 else 0
+    if wsb:
+        ws = _workspace(wsb, x.device)
+        st = lib.catopt_hip_linear_ws(dt, M, N, K, _ptr(x2), ldx, _ptr(weight), weight.stride(0), _ptr(bias),
+                                      _ptr(bias2), int(epilogue), _ptr(y), N, _ptr(ws), wsb, _stream(x))
+    else:
+        st = lib.catopt_hip_linear(dt, M, N, K, _ptr(x2), ldx, _ptr(weight), weight.stride(0),
+                                   _ptr(bias), _ptr(bias2), int(epilogue), _ptr(y), N, _stream(x))
     L.check("catopt_hip_linear", st)
     return y
 

@@ -100,8 +100,8 @@ int32_t catopt_hip_rmsnorm(int32_t dtype, int64_t rows, int64_t cols,
  * two projections, first half then second half).  bias / bias2 are [N]
  * vectors of `dtype` (NULL unless the epilogue reads them).  fp32
  * accumulation.  bf16 with K-contiguous, 16-byte aligned operands and
- * K % 8 == 0 runs the persistent 16x16x32 bf16 MFMA kernel (one workgroup
- * per CU); other bf16 and all fp32 calls run 32x32x2 fp32 MFMA kernels.
+ * K % 8 == 0 runs the 16x16x32 bf16 MFMA kernels (few rows, middle or large
+ * tiles, by size); other bf16 and all fp32 calls run fp32 MFMA kernels.
  * Replaces the "linear" binding (torch_bridge.py:1251-1253), the bias adds
  * of the ASSOC_LINEAR_BIAS RHS (laws/tensor.py:1374-1394), and the
  * chunk/silu/mul (or glu) bindings of the SWIGLU_FUSE / GLU_FOLD RHS
@@ -112,6 +112,22 @@ int32_t catopt_hip_linear(int32_t dtype, int64_t M, int64_t N, int64_t K,
                           int64_t ldw, const void* bias, const void* bias2,
                           int32_t epilogue, void* y, int64_t ldy,
                           void* stream);
+
+/*
+ * catopt_hip_linear with a workspace: bf16 products whose tiles do not fill
+ * the chip then split K and add the ranges' fp32 partial sums in a fixed
+ * order (the workspace holds them).  catopt_hip_linear_workspace_bytes is
+ * the size such a call reads on the current device (0: none, -1: invalid
+ * arguments); with less, or NULL, the call runs without splitting K.
+ */
+int64_t catopt_hip_linear_workspace_bytes(int32_t dtype, int64_t M, int64_t N,
+                                          int64_t K, int32_t epilogue);
+int32_t catopt_hip_linear_ws(int32_t dtype, int64_t M, int64_t N, int64_t K,
+                             const void* x, int64_t ldx, const void* w,
+                             int64_t ldw, const void* bias, const void* bias2,
+                             int32_t epilogue, void* y, int64_t ldy,
+                             void* workspace, int64_t workspace_bytes,
+                             void* stream);
 
 /*
  * Batched matrix product with optional transposes:

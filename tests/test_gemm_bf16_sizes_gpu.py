@@ -72,6 +72,40 @@ def test_linear_sizes(M, N, Kd, epi, pad):
     _check(y, *_reference(x, w, epi, bias, bias2))
 
 
+# the middle tiles: one row past the few-row kernels, tile edges either side,
+# whole tiles only, K ranges (with a K tail), a last round split in ranges, odd N
+MID = [(65, 256, 4096), (64, 1024, 4104), (128, 4096, 1032), (129, 130, 2056), (200, 1003, 2048), (333, 640, 5000),
+       (257, 4096, 520), (400, 11008, 72), (1000, 2752, 264), (300, 11010, 1024)]
+
+
+@pytest.mark.parametrize("epi", [L.EPI_NONE, L.EPI_BIAS, L.EPI_BIAS_ADD2, L.EPI_SILU_MUL, L.EPI_GLU])
+@pytest.mark.parametrize("M,N,Kd", MID)
+def test_linear_middle_sizes(M, N, Kd, epi):
+    test_linear_sizes(M, N, Kd, epi, 16 if M % 2 else 0)
+
+
+@pytest.mark.parametrize("epi", [L.EPI_BIAS, L.EPI_GLU])
+def test_linear_without_workspace_and_with_too_little(epi):
+    """The same product from every workspace the entry point may be given."""
+    M, N, Kd = 100, 512, 4096
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn((M, Kd), generator=g, device=DEV).to(BF)
+    w = torch.randn((2 * N if epi == L.EPI_GLU else N, Kd), generator=g, device=DEV).to(BF)
+    bias = torch.randn(N, generator=g, device=DEV).to(BF) if epi == L.EPI_BIAS else None
+    lib = L.load()
+    need = lib.catopt_hip_linear_workspace_bytes(L.BF16, M, N, Kd, epi)
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    ref = _reference(x, w, epi, bias, None)
+    for p, n in ((None, 0), (ws.data_ptr(), need - 1), (ws.data_ptr(), need)):
+        y = torch.empty((M, N), dtype=BF, device=DEV)
+        st = lib.catopt_hip_linear_ws(L.BF16, M, N, Kd, x.data_ptr(), Kd, w.data_ptr(), Kd,
+                                      None if bias is None else bias.data_ptr(), None, epi, y.data_ptr(), N, p, n,
+                                      torch.cuda.current_stream().cuda_stream)
+        assert st == L.OK
+        _check(y, *ref)
+
+
 @pytest.mark.parametrize("nb,M,N,Kd", [(3, 1, 40, 64), (5, 20, 96, 136), (2, 64, 33, 256)])
 def test_batched_few_rows(nb, M, N, Kd):
     g = torch.Generator(device=DEV).manual_seed(nb + M)
