@@ -16,6 +16,8 @@
 //             This is the two-level blocked scan of the reference's
 //             all-prefix path; it trades a second read of the inputs for
 //             chunk-level parallelism when B*D*N alone cannot fill the GPU.
+// The selective SSM scan streams in T-segments of its own choosing instead
+// (ssm_segment below); only an explicit CHUNKED schedule walks the table.
 #include <mutex>
 
 #include "common.hpp"
@@ -167,10 +169,24 @@ __device__ __forceinline__ void ssm_load(SsmStep<N, APS>& st, const float* __res
   st.x = x[bt * D + d];
 }
 
+// p plus the DPP-moved p of another lane.
+template <int CTRL>
+__device__ __forceinline__ float add_dpp(float p) {
+  return p + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(p), CTRL, 0xf, 0xf, true));
+}
+
+// The sum over the TPD lanes of a channel, on every one of them: quad
+// permutations (lane ^ 1, lane ^ 2), then the mirror of 8 and of 16 lanes,
+// whose halves are uniform by then.  A shuffle through LDS per level put
+// four LDS latencies on every step of the streaming scan: 0.21 us a step.
 template <int N>
 __device__ __forceinline__ float lane_reduce(float p) {
-#pragma unroll
-  for (int o = 1; o < SsmLayout<N>::TPD; o <<= 1) p += __shfl_xor(p, o, 64);
+  constexpr int TPD = SsmLayout<N>::TPD;
+  static_assert(TPD <= 16, "a channel's lanes lie in one DPP row");
+  if (TPD >= 2) p = add_dpp<0xB1>(p);    // quad_perm [1, 0, 3, 2]
+  if (TPD >= 4) p = add_dpp<0x4E>(p);    // quad_perm [2, 3, 0, 1]
+  if (TPD >= 8) p = add_dpp<0x141>(p);   // row_half_mirror
+  if (TPD >= 16) p = add_dpp<0x140>(p);  // row_mirror
   return p;
 }
 
@@ -245,22 +261,6 @@ __device__ __forceinline__ SsmIdx<N> ssm_idx(int64_t D) {
 }
 
 template <int N, bool APS>
-__global__ __launch_bounds__(kThreads) void ssm_stream(
-    const float* __restrict__ a, const float* __restrict__ bx, const float* __restrict__ c,
-    const float* __restrict__ x, const float* __restrict__ h0, const int64_t* __restrict__ cs,
-    int64_t nc, int64_t T, int64_t D, float* __restrict__ y, float* __restrict__ hf) {
-  const SsmIdx<N> ix = ssm_idx<N>(D);
-  const int64_t b = blockIdx.y;
-  f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int64_t sidx = (b * D + ix.d) * N + ix.n0;
-  if (h0 && ix.dok) h = *reinterpret_cast<const f32x4*>(h0 + sidx);
-  for (int64_t k = 0; k < nc; ++k)
-    h = ssm_run<N, APS, true>(a, bx, c, x, y, b, T, D, ix.d, ix.dok, ix.n0, cclamp(cs[k], T),
-                              cclamp(cs[k + 1], T), h, nullptr);
-  if (hf && ix.dok) *reinterpret_cast<f32x4*>(hf + sidx) = h;
-}
-
-template <int N, bool APS>
 __global__ __launch_bounds__(kThreads) void ssm_chunk_local(
     const float* __restrict__ a, const float* __restrict__ bx, const float* __restrict__ c,
     const float* __restrict__ x, const int64_t* __restrict__ cs, int64_t T, int64_t D,
@@ -290,264 +290,231 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_apply(
                         cclamp(cs[k + 1], T), h, nullptr);
 }
 
-// ----------------------------------------------------- LDS-staged streaming
-// The streaming schedule for a per-state a (B, T, D, N), fed through LDS:
-// a workgroup owns DPW channels x N states (one 4 KB slice of a per step)
-// and streams U-step stages of a, b, c and x into LDS with direct
-// global->LDS loads (no registers held while the loads are in flight), two
-// stages deep: the loads of stage s+1 are issued before the arithmetic of
-// stage s and waited for after it, one barrier per stage.  Each workgroup
-// thus keeps U x ~4.4 KB of reads in flight, two workgroups per CU, which is
-// what HBM's bandwidth-latency product asks of 256 CUs.  The chunk table
-// tiles [0, T) in order, so one pass over t = 0 .. T-1 is that walk.
-constexpr int SU = 8;  // steps per LDS stage
-
-template <int N>
-struct SsmLds {
-  static constexpr int TPD = N / 4, DPW = kThreads / TPD;
-  static constexpr int A_BYTES = SU * DPW * N * 4;   // SU x 4 KB
-  static constexpr int X_BYTES = SU * DPW * 4;
-  static constexpr int V_BYTES = SU * N * 4;         // b or c
-  static constexpr int STAGE = A_BYTES + X_BYTES + 2 * V_BYTES;
-  static constexpr int BYTES = 2 * STAGE;
-  static constexpr int X_SLOTS = SU * DPW;           // 4-byte slots
-  static constexpr int V_SLOTS = SU * N;
-};
-
-typedef __attribute__((address_space(3))) void* lds_vptr;
-
-template <int N>
-__global__ __launch_bounds__(kThreads, 2) void ssm_stream_lds(
-    const float* __restrict__ a, const float* __restrict__ bx, const float* __restrict__ c,
-    const float* __restrict__ x, const float* __restrict__ h0, int64_t T, int64_t D,
-    float* __restrict__ y, float* __restrict__ hf) {
-  using L = SsmLds<N>;
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t b = blockIdx.y;
-  const int64_t d0 = (int64_t)blockIdx.x * L::DPW;
-  const int ch = tid / L::TPD, n0 = (tid % L::TPD) * 4;
-  const int64_t d = d0 + ch;
-  const bool dok = d < D;
-  // a slot of this thread: channel d (clamped to a valid one), states n0..n0+3
-  const int64_t a_lane = (((dok ? d : D - 1) * N) + n0);
-  const int64_t nst = (T + SU - 1) / SU;
-
-  auto issue = [&](int64_t st, int stage) {
-    char* base = lds + stage * L::STAGE;
-    const int64_t t0 = st * SU;
-#pragma unroll
-    for (int u = 0; u < SU; ++u) {
-      const int64_t t = t0 + u < T ? t0 + u : T - 1;
-      const float* src = a + ((b * T + t) * D) * N + a_lane;
-      __builtin_amdgcn_global_load_lds(src, (lds_vptr)(base + u * (L::DPW * N * 4) + wave * 1024), 16, 0, 0);
-    }
-    char* xb = base + L::A_BYTES;
-#pragma unroll
-    for (int i = 0; i < (L::X_SLOTS + kThreads - 1) / kThreads; ++i) {
-      const int s = i * kThreads + tid;
-      if (i * kThreads + wave * 64 < L::X_SLOTS) {  // whole waves: DPW*SU is a multiple of 64
-        const int u = s / L::DPW, cc = s % L::DPW;
-        const int64_t t = t0 + u < T ? t0 + u : T - 1;
-        const int64_t dd = d0 + cc < D ? d0 + cc : D - 1;
-        __builtin_amdgcn_global_load_lds(x + (b * T + t) * D + dd,
-                                         (lds_vptr)(xb + (i * kThreads + wave * 64) * 4), 4, 0, 0);
-      }
-    }
-    char* vb = xb + L::X_BYTES;
-#pragma unroll
-    for (int i = 0; i < (L::V_SLOTS + kThreads - 1) / kThreads; ++i) {
-      const int s = i * kThreads + tid;
-      if (s < L::V_SLOTS) {
-        const int u = s / N, n = s % N;
-        const int64_t t = t0 + u < T ? t0 + u : T - 1;
-        const int64_t off = (b * T + t) * N + n;
-        const int lbase = (i * kThreads + wave * 64) * 4;
-        __builtin_amdgcn_global_load_lds(bx + off, (lds_vptr)(vb + lbase), 4, 0, 0);
-        __builtin_amdgcn_global_load_lds(c + off, (lds_vptr)(vb + L::V_BYTES + lbase), 4, 0, 0);
-      }
-    }
-  };
-
-  f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int64_t sidx = (b * D + (dok ? d : 0)) * N + n0;
-  if (h0 && dok) h = *reinterpret_cast<const f32x4*>(h0 + sidx);
-  if (nst > 0) {
-    issue(0, 0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  }
-  for (int64_t st = 0; st < nst; ++st) {
-    const int cur = (int)(st & 1);
-    if (st + 1 < nst) issue(st + 1, cur ^ 1);
-    const char* base = lds + cur * L::STAGE;
-    const char* xb = base + L::A_BYTES;
-    const char* vb = xb + L::X_BYTES;
-    const int64_t t0 = st * SU;
-    const int un = T - t0 < SU ? (int)(T - t0) : SU;
-    for (int u = 0; u < un; ++u) {
-      const f32x4 av = *reinterpret_cast<const f32x4*>(base + u * (L::DPW * N * 4) + tid * 16);
-      const f32x4 bv = *reinterpret_cast<const f32x4*>(vb + (u * N + n0) * 4);
-      const f32x4 cv = *reinterpret_cast<const f32x4*>(vb + L::V_BYTES + (u * N + n0) * 4);
-      const float xv = *reinterpret_cast<const float*>(xb + (u * L::DPW + ch) * 4);
-      h = av * h + bv * xv;
-      const f32x4 chv = cv * h;
-      const float r = lane_reduce<N>(chv[0] + chv[1] + chv[2] + chv[3]);
-      if (dok && n0 == 0) y[(b * T + t0 + u) * D + d] = r;
-    }
-    if (st + 1 < nst) {
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-    }
-  }
-  if (hf && dok) *reinterpret_cast<f32x4*>(hf + sidx) = h;
-}
-
-// --------------------------------------------------- register-staged streaming
-// The streaming schedule for a per-state a (N = 16) with a held in registers:
-// each thread's 16-byte slices of a for RSU steps go straight into one of
-// two register sets while the other set's steps run; the small x, b and c
-// streams go through LDS (one copy per workgroup) by direct loads issued
-// before a's, and y leaves through LDS as whole rows.  Every wave issues the
-// same memory operations in every stage with no branch around them, so the
+// ------------------------------------------------------- streaming segments
+// The scan over T-segments: a workgroup owns DPW channels x N states (one
+// 4 KB slice of a per step, 16 bytes per thread) and walks one segment of
+// the steps.  With one segment (enough workgroups to fill the chip) that is
+// a single pass over a; with P segments two launches:
+//   EMIT = false  composes each segment but the last into (prod a, local
+//                 state), reading a, b and x;
+//   EMIT = true   starts each segment from h0 folded through the segments
+//                 before it, and emits y.
+// HBM bounds both, and below two workgroups per CU what bounds a workgroup
+// is the latency of its loads: with loads one stage ahead a stage took 1.66 us
+// (20 GB/s per workgroup).  So everything is loaded two stages ahead: a's
+// slices for RSU steps go straight into one of three register sets, the
+// small x, b and c streams through LDS (one copy per workgroup, three
+// buffers) by direct loads issued before a's, and y leaves through LDS as
+// whole rows.  The loads have no lane-dependent branch around them, so the
 // waits the compiler derives for a are exact, and the wait at the end of a
-// stage leaves the RSU newest loads (the next stage's a) in flight across
-// the barrier: two stages of a (2 x RSU x 4 KB per workgroup) stay in
-// flight and no stage drains the memory pipeline.  On gfx9 stores count in
-// vmcnt too, which is why y is not stored step by step under a lane mask.
-// y's stores are non-temporal (written once, never read back here): 1.5%
-// faster at C5's shape than plain stores.  What y costs beyond that is
-// HBM's turnaround between reads and writes; a plain streaming kernel with
-// the same 16:1 read/write mix pays it as well.  Steps past the last whole
-// stage run unpipelined.  (The LDS-staged kernel above waits for all its
-// loads at every stage, which measured 5-14% slower at C5's shape.)
+// stage leaves the newest 2 RSU operations in flight across the barrier: it
+// covers the next stage's small streams, which are older than its a.  On
+// gfx9 stores count in vmcnt too, which is why y is not stored step by step
+// under a lane mask.  y's stores are non-temporal (written once, never read
+// back here): 1.5% faster at C5's shape than plain stores.  What y costs
+// beyond that is HBM's turnaround between reads and writes; a plain
+// streaming kernel with the same 16:1 read/write mix pays it as well.  Steps
+// past the last whole stage run unpipelined.
 #ifndef CATOPT_SSM_RSU
 #define CATOPT_SSM_RSU 8
 #endif
-constexpr int RSU = CATOPT_SSM_RSU;  // steps per stage of the register-staged scan
+constexpr int RSU = CATOPT_SSM_RSU;  // steps per stage
 
 template <int N>
 struct SsmSmall {
   static constexpr int TPD = N / 4, DPW = kThreads / TPD;
-  static constexpr int X_BYTES = RSU * DPW * 4;
-  static constexpr int V_BYTES = RSU * N * 4;   // b or c
-  static constexpr int STAGE = X_BYTES + 2 * V_BYTES;
-  static constexpr int Y_BYTES = RSU * DPW * 4;
-  static constexpr int BYTES = 2 * STAGE + 2 * Y_BYTES;
-  static constexpr int XPT = RSU * DPW / kThreads;         // x loads (and y stores) per thread
-  static constexpr int VPT = 2 * RSU * N / kThreads;       // b and c loads per thread
-  static_assert(RSU * DPW % kThreads == 0 && 2 * RSU * N % kThreads == 0, "whole waves per small stream");
-  static_assert(RSU * N % 64 == 0, "b and c slots in whole waves");
+  static constexpr int X_SLOTS = RSU * DPW, V_SLOTS = 2 * RSU * N;  // 4-byte slots: x (and y); b, then c
+  static constexpr int STAGE = (X_SLOTS + V_SLOTS) * 4;
+  static constexpr int Y_BYTES = X_SLOTS * 4;
+  static constexpr int BYTES = 3 * (STAGE + Y_BYTES);
+  static constexpr int XPT = (X_SLOTS + kThreads - 1) / kThreads;  // x loads (and y stores) per thread
+  static constexpr int VPT = (V_SLOTS + kThreads - 1) / kThreads;  // b and c loads per thread
+  static_assert(X_SLOTS % 64 == 0 && V_SLOTS % 64 == 0, "whole waves per small stream");
 };
 
-template <int N>
-__global__ __launch_bounds__(kThreads, 2) void ssm_stream_reg(
+// The stages [first, second) of RSU steps that segment seg of P walks (the
+// steps past the last whole stage belong to the last segment).
+__device__ __forceinline__ int64_t seg_stage(int64_t T, int64_t seg, int64_t P) { return (T / RSU) * seg / P; }
+
+// a ⊙ h + b x, rounding a h and fusing b x: with a in (0, 1) the rounded
+// product is the smaller one, and the states' error against 64 bits is 12%
+// less than with the other product rounded.
+__device__ __forceinline__ f32x4 ssm_step(f32x4 a, f32x4 h, f32x4 b, float x) {
+  const f32x4 ah = a * h;
+  f32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __builtin_fmaf(b[i], x, ah[i]);
+  return r;
+}
+
+template <int N, bool APS, bool EMIT>
+__global__ __launch_bounds__(kThreads, 2) void ssm_segment(
     const float* __restrict__ a, const float* __restrict__ bx, const float* __restrict__ c,
-    const float* __restrict__ x, const float* __restrict__ h0, int64_t T, int64_t D,
-    float* __restrict__ y, float* __restrict__ hf) {
+    const float* __restrict__ x, const float* __restrict__ h0, int64_t T, int64_t D, int64_t S,
+    int64_t P, float* __restrict__ ws_p, float* __restrict__ ws_h, float* __restrict__ y,
+    float* __restrict__ hf) {
   using L = SsmSmall<N>;
   __shared__ __attribute__((aligned(16))) char lds[L::BYTES];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t b = blockIdx.y;
+  const int64_t b = blockIdx.y, seg = blockIdx.z;
   const int64_t d0 = (int64_t)blockIdx.x * L::DPW;
   const int ch = tid / L::TPD, n0 = (tid % L::TPD) * 4;
   const int64_t d = d0 + ch;
   const bool dok = d < D;
-  const int64_t a_lane = (((dok ? d : D - 1) * N) + n0);
-  const int64_t nfull = T / RSU;
-  // this thread's small-stream slots: x (u, channel) for two slots; b (waves
-  // 0, 1) or c (waves 2, 3) for one (u, n) slot, clamped to valid rows
-  int xu[L::XPT], xc[L::XPT];
+  const int64_t dd = dok ? d : D - 1;  // channels past D shadow the last one, never stored
+  const int64_t st0 = seg_stage(T, seg, P), st1 = seg_stage(T, seg + 1, P);
+  // this thread's x slots (step u, channel), clamped to valid channels: their
+  // elements' offsets in a stage of x and of y, and their words in LDS.  All
+  // per-stage address arithmetic is on wave-uniform bases.
+  int64_t xo[L::XPT];
+  int xw[L::XPT];
 #pragma unroll
   for (int i = 0; i < L::XPT; ++i) {
-    const int s = i * kThreads + tid;
-    xu[i] = s / L::DPW;
-    xc[i] = (int)(d0 + s % L::DPW < D ? s % L::DPW : D - 1 - d0);
+    const int s = i * kThreads + tid, u = s / L::DPW;
+    const int cc = (int)(d0 + s % L::DPW < D ? s % L::DPW : D - 1 - d0);
+    xo[i] = u * D + d0 + cc;
+    xw[i] = u * L::DPW + cc;
   }
+  const uint32_t ao = (uint32_t)(APS ? (dd - d0) * N + n0 : dd - d0);
 
   const uint32_t lds0 = lds_u32(lds);
+  // the guards are wave-uniform: every stream is a whole number of waves
   auto issue_small = [&](int64_t st, int stage) {
     const uint32_t xb = lds0 + stage * L::STAGE;
-    const int64_t t0 = st * RSU;
+    const int64_t bt = b * T + st * RSU;
+    const float* xr = x + bt * D;
 #pragma unroll
     for (int i = 0; i < L::XPT; ++i)
-      dma4(x + (b * T + t0 + xu[i]) * D + d0 + xc[i], xb + (i * kThreads + wave * 64) * 4);
+      if (i * kThreads + wave * 64 < L::X_SLOTS) dma4(xr + xo[i], xb + (i * kThreads + wave * 64) * 4);
     // b then c, one 4-byte slot per lane: slots [0, RSU*N) of b, then of c
+    // (not emitting, b alone)
 #pragma unroll
     for (int i = 0; i < L::VPT; ++i) {
       const int s = i * kThreads + tid;
-      const bool is_c = s >= RSU * N;              // wave-uniform: RSU*N is a multiple of 64
-      const int vs = is_c ? s - RSU * N : s;
-      dma4((is_c ? c : bx) + (b * T + t0 + vs / N) * N + vs % N,
-           __builtin_amdgcn_readfirstlane(xb + L::X_BYTES + (is_c ? L::V_BYTES : 0) + (vs & ~63) * 4));
+      if (i * kThreads + wave * 64 < (EMIT ? L::V_SLOTS : L::V_SLOTS / 2)) {
+        const bool is_c = s >= RSU * N;
+        dma4((is_c ? c : bx) + bt * N + (is_c ? s - RSU * N : s), xb + (L::X_SLOTS + i * kThreads + wave * 64) * 4);
+      }
     }
   };
   auto load_a = [&](int64_t st, f32x4* ra) {
-    const int64_t t0 = st * RSU;
+    const float* ar = a + ((b * T + st * RSU) * D + d0) * (APS ? N : 1);
+    const int64_t row = D * (APS ? N : 1);
 #pragma unroll
-    for (int u = 0; u < RSU; ++u)
-      ra[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(a + ((b * T + t0 + u) * D) * N + a_lane));
+    for (int u = 0; u < RSU; ++u) {
+      if (APS) {
+        ra[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(ar + u * row + ao));
+      } else {
+        const float av = (ar + u * row)[ao];
+        ra[u] = f32x4{av, av, av, av};
+      }
+    }
   };
 
-  f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int64_t sidx = (b * D + (dok ? d : 0)) * N + n0;
-  if (h0 && dok) h = *reinterpret_cast<const f32x4*>(h0 + sidx);
+  f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f}, p = f32x4{1.f, 1.f, 1.f, 1.f};
+  const int64_t sidx = (b * D + dd) * N + n0;
+  if (EMIT) {
+    if (h0) h = *reinterpret_cast<const f32x4*>(h0 + sidx);
+    // the segments before this one, in order; their summaries do not depend
+    // on the carry, so a batch of them costs one memory latency
+    constexpr int kBatch = 8;
+    for (int64_t k0 = 0; k0 < seg; k0 += kBatch) {
+      f32x4 pk[kBatch], hk[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i)
+        if (k0 + i < seg) {
+          pk[i] = *reinterpret_cast<const f32x4*>(ws_p + (k0 + i) * S + sidx);
+          hk[i] = *reinterpret_cast<const f32x4*>(ws_h + (k0 + i) * S + sidx);
+        }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i)
+        if (k0 + i < seg) h = pk[i] * h + hk[i];
+    }
+  }
   auto compute = [&](int stage, const f32x4* ra, char* yb) {
     const char* xb = lds + stage * L::STAGE;
-    const char* vb = xb + L::X_BYTES;
+    const char* vb = xb + L::X_SLOTS * 4;
+    float r[RSU];
 #pragma unroll
     for (int u = 0; u < RSU; ++u) {
       const f32x4 bv = *reinterpret_cast<const f32x4*>(vb + (u * N + n0) * 4);
-      const f32x4 cv = *reinterpret_cast<const f32x4*>(vb + L::V_BYTES + (u * N + n0) * 4);
       const float xv = *reinterpret_cast<const float*>(xb + (u * L::DPW + ch) * 4);
-      h = ra[u] * h + bv * xv;
-      const f32x4 chv = cv * h;
-      const float r = lane_reduce<N>(chv[0] + chv[1] + chv[2] + chv[3]);
-      if (n0 == 0) *reinterpret_cast<float*>(yb + (u * L::DPW + ch) * 4) = r;
+      h = ssm_step(ra[u], h, bv, xv);
+      if (EMIT) {
+        const f32x4 cv = *reinterpret_cast<const f32x4*>(vb + (RSU * N + u * N + n0) * 4);
+        const f32x4 chv = cv * h;
+        r[u] = lane_reduce<N>(chv[0] + chv[1] + chv[2] + chv[3]);
+      } else {
+        p *= ra[u];
+      }
+    }
+    if (!EMIT) return;
+    // every lane of a channel has every step's sum: lane j writes steps j,
+    // j + TPD, ... (a write under a lane mask per step would keep the next
+    // step's reads from being issued ahead of it)
+    const int j = (tid % L::TPD) % RSU;
+#pragma unroll
+    for (int k = 0; k < RSU; k += L::TPD) {
+      float v = r[k];
+#pragma unroll
+      for (int i = 1; i < L::TPD && i < RSU; ++i) v = j == i ? r[k + i] : v;
+      *reinterpret_cast<float*>(yb + ((k + j) * L::DPW + ch) * 4) = v;
     }
   };
   // y rows of a stage from LDS: row u, channels d0 .. d0 + DPW - 1
   auto store_y = [&](int64_t st, const char* yb) {
+    float* yr = y + (b * T + st * RSU) * D;
 #pragma unroll
     for (int i = 0; i < L::XPT; ++i) {
       // a channel past D (last, partial workgroup) writes channel D - 1's
       // value to it again: no lane mask around the store
-      const int u = (i * kThreads + tid) / L::DPW;
-      const int cc = xc[i];  // the clamped channel of slot i
-      __builtin_nontemporal_store(*reinterpret_cast<const float*>(yb + (u * L::DPW + cc) * 4),
-                                  y + (b * T + st * RSU + u) * D + d0 + cc);
+      if (i * kThreads + wave * 64 < L::X_SLOTS)
+        __builtin_nontemporal_store(*reinterpret_cast<const float*>(yb + xw[i] * 4), yr + xo[i]);
     }
   };
-  char* ybuf0 = lds + 2 * L::STAGE;
-  char* ybuf1 = ybuf0 + L::Y_BYTES;
-  auto step = [&](int64_t st, int buf, f32x4* cur, f32x4* nxt) {
-    const int64_t sn = st + 1 < nfull ? st + 1 : nfull - 1;  // the last stage reloads itself
-    issue_small(sn, buf ^ 1);
-    load_a(sn, nxt);
-    char* yb = buf ? ybuf1 : ybuf0;
+  // vmcnt <= 2 RSU, lgkmcnt 0
+  auto landed = [&]() {
+    __builtin_amdgcn_s_waitcnt((2 * RSU & 15) | (7 << 4) | ((2 * RSU >> 4) << 14));
+    __syncthreads();
+  };
+  auto issue = [&](int64_t st, int buf, f32x4* ra) {
+    const int64_t sn = st < st1 ? st : st1 - 1;  // past the end: the last stage again, not read
+    issue_small(sn, buf);
+    load_a(sn, ra);
+  };
+  // stage st from buffer and register set `buf`, stage st + 2 into `ahead`
+  auto step = [&](int64_t st, int buf, const f32x4* cur, int ahead, f32x4* nxt) {
+    issue(st + 2, ahead, nxt);
+    char* yb = lds + 3 * L::STAGE + buf * L::Y_BYTES;
     compute(buf, cur, yb);
-    __builtin_amdgcn_s_waitcnt((RSU & 15) | (7 << 4) | ((RSU >> 4) << 14));  // vmcnt <= RSU, lgkmcnt 0
-    __syncthreads();
-    store_y(st, yb);
+    landed();
+    if (EMIT) store_y(st, yb);
   };
-  f32x4 ra0[RSU], ra1[RSU];
-  if (nfull > 0) {
-    issue_small(0, 0);
-    load_a(0, ra0);
-    __builtin_amdgcn_s_waitcnt((RSU & 15) | (7 << 4) | ((RSU >> 4) << 14));
-    __syncthreads();
-    for (int64_t st = 0; st < nfull; st += 2) {
-      step(st, 0, ra0, ra1);
-      if (st + 1 < nfull) step(st + 1, 1, ra1, ra0);
+  f32x4 ra0[RSU], ra1[RSU], ra2[RSU];
+  if (st0 < st1) {
+    issue(st0, 0, ra0);
+    issue(st0 + 1, 1, ra1);
+    landed();
+    for (int64_t st = st0; st < st1; st += 3) {
+      step(st, 0, ra0, 2, ra2);
+      if (st + 1 < st1) step(st + 1, 1, ra1, 0, ra0);
+      if (st + 2 < st1) step(st + 2, 2, ra2, 1, ra1);
     }
+    __builtin_amdgcn_s_waitcnt(0);  // the loads past the end have landed in LDS
   }
+  if (!EMIT) {
+    if (!dok) return;
+    *reinterpret_cast<f32x4*>(ws_p + seg * S + sidx) = p;
+    *reinterpret_cast<f32x4*>(ws_h + seg * S + sidx) = h;
+    return;
+  }
+  if (seg + 1 < P) return;
   // steps past the last whole stage
-  for (int64_t t = nfull * RSU; t < T; ++t) {
-    SsmStep<N, true> sp;
-    ssm_load(sp, a, bx, c, x, b, t, T, D, dok ? d : 0, n0);
-    h = sp.a * h + sp.bx * sp.x;
+  for (int64_t t = T / RSU * RSU; t < T; ++t) {
+    SsmStep<N, APS> sp;
+    ssm_load(sp, a, bx, c, x, b, t, T, D, dd, n0);
+    h = ssm_step(sp.a, h, sp.bx, sp.x);
     const f32x4 chv = sp.c * h;
     const float r = lane_reduce<N>(chv[0] + chv[1] + chv[2] + chv[3]);
     if (dok && n0 == 0) y[(b * T + t) * D + d] = r;
@@ -566,15 +533,31 @@ bool affd_chunked(int64_t S, int64_t nc, int32_t schedule) {
   return schedule == CATOPT_SCAN_AUTO && nc > 1 && S < kFillThreads;
 }
 
-int64_t ssm_threads(int64_t B, int64_t D, int64_t N) {
-  const int64_t tpd = N / 4;  // threads per channel (4 states per thread)
-  const int64_t dpw = kThreads / tpd;
-  return (D + dpw - 1) / dpw * kThreads * B;
+// Segments of the SSM scan under the automatic schedule, at most one per chunk
+// of the caller's table (which sizes the workspace).  One pass reads a once
+// but takes 0.86 us per stage however few workgroups walk it; P segments read
+// it 2 - 1/P times.  One pass wins from about 84 workgroups up (D = 2048,
+// N = 16, T = 8192: 128 workgroups 1033 us against 1307 at P = 2, 64
+// workgroups 906 against 701 at P = 4).  Below that the best P puts one
+// workgroup on each CU: more, and the pass ends in a part-filled second round
+// (32 workgroups, T = 8192: P = 8 365 us, P = 10 438, P = 16 396).  Many
+// segments are taken odd in number, so that their starts do not lie a power
+// of two of bytes apart (16 workgroups, T = 2048: P = 15 50 us, P = 16 61).
+int64_t ssm_segments(int64_t B, int64_t T, int64_t D, int64_t N, int64_t nc) {
+  constexpr int64_t kOnePass = 84, kCus = 256, kMinStages = 2;
+  const int64_t dpw = kThreads / (N / 4);  // channels per workgroup
+  const int64_t wgs = (D + dpw - 1) / dpw * B;
+  if (wgs <= 0 || wgs >= kOnePass || nc <= 1) return 1;
+  int64_t P = kCus / wgs;
+  if (P > 8 && P % 2 == 0) --P;
+  if (P > T / (RSU * kMinStages)) P = T / (RSU * kMinStages);
+  if (P > nc) P = nc;
+  return P < 2 ? 1 : P;
 }
 
-bool ssm_chunked(int64_t B, int64_t D, int64_t N, int64_t nc, int32_t schedule) {
+bool ssm_chunked(int64_t B, int64_t T, int64_t D, int64_t N, int64_t nc, int32_t schedule) {
   if (schedule == CATOPT_SCAN_CHUNKED) return true;
-  return schedule == CATOPT_SCAN_AUTO && nc > 1 && ssm_threads(B, D, N) < kFillThreads;
+  return schedule == CATOPT_SCAN_AUTO && ssm_segments(B, T, D, N, nc) > 1;
 }
 
 template <int N, bool APS>
@@ -584,32 +567,20 @@ int32_t ssm_launch(int64_t B, int64_t T, int64_t D, const float* a, const float*
                    hipStream_t s) {
   const int64_t gx = (D + SsmLayout<N>::DPW - 1) / SsmLayout<N>::DPW;
   const int64_t S = B * D * N;
-  static_assert(SsmLayout<N>::TPD == N / 4, "ssm_threads assumes four states per thread");
-  const bool chunked = ssm_chunked(B, D, N, nc, schedule);
+  static_assert(SsmLayout<N>::TPD == N / 4, "ssm_segments assumes four states per thread");
   if (gx > 0x7fffffff || B > 65535 || nc > 65535) return CATOPT_E_UNSUPPORTED;
-  if constexpr (N == 16) {
-    if (!chunked && APS) {
-      ssm_stream_reg<N><<<dim3((uint32_t)gx, (uint32_t)B), dim3(kThreads), 0, s>>>(a, bx, c, x, h0, T, D, y, hf);
+  if (schedule != CATOPT_SCAN_CHUNKED) {
+    int64_t P = schedule == CATOPT_SCAN_AUTO ? ssm_segments(B, T, D, N, nc) : 1;
+    float* ws_p = static_cast<float*>(ws);
+    float* ws_h = ws_p + P * S;
+    if (P > 1) {
+      if (!ws || wsb < catopt_hip_scan_workspace_bytes(S, nc)) return CATOPT_E_WORKSPACE;
+      ssm_segment<N, APS, false><<<dim3((uint32_t)gx, (uint32_t)B, (uint32_t)(P - 1)), dim3(kThreads), 0, s>>>(
+          a, bx, c, x, h0, T, D, S, P, ws_p, ws_h, y, hf);
       CATOPT_LAUNCH_CHECK();
-      return CATOPT_OK;
     }
-  }
-  if (!chunked && APS) {
-    static bool attr_done = false;
-    if (!attr_done) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_stream_lds<N>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, SsmLds<N>::BYTES);
-      if (e != hipSuccess) return set_hip_error(e);
-      attr_done = true;
-    }
-    ssm_stream_lds<N><<<dim3((uint32_t)gx, (uint32_t)B), dim3(kThreads), SsmLds<N>::BYTES, s>>>(
-        a, bx, c, x, h0, T, D, y, hf);
-    CATOPT_LAUNCH_CHECK();
-    return CATOPT_OK;
-  }
-  if (!chunked) {
-    ssm_stream<N, APS><<<dim3((uint32_t)gx, (uint32_t)B), dim3(kThreads), 0, s>>>(
-        a, bx, c, x, h0, cs, nc, T, D, y, hf);
+    ssm_segment<N, APS, true><<<dim3((uint32_t)gx, (uint32_t)B, (uint32_t)P), dim3(kThreads), 0, s>>>(
+        a, bx, c, x, h0, T, D, S, P, ws_p, ws_h, y, hf);
     CATOPT_LAUNCH_CHECK();
     return CATOPT_OK;
   }
@@ -650,7 +621,7 @@ extern "C" int64_t catopt_hip_ssm_scan_workspace_bytes(int64_t B, int64_t T, int
   if (B < 0 || T < 0 || D < 0 || n_chunks < 1) return -1;
   if (schedule < CATOPT_SCAN_AUTO || schedule > CATOPT_SCAN_CHUNKED) return -1;
   if (N != 4 && N != 8 && N != 16 && N != 32 && N != 64) return -1;
-  return ssm_chunked(B, D, N, n_chunks, schedule) ? catopt_hip_scan_workspace_bytes(B * D * N, n_chunks)
+  return ssm_chunked(B, T, D, N, n_chunks, schedule) ? catopt_hip_scan_workspace_bytes(B * D * N, n_chunks)
                                                   : 0;
 }
 
