@@ -50,7 +50,7 @@
 // tracked separately so the emitted (m, l, a) carrier is the om_elem one.
 #include <type_traits>
 
-#include "common.hpp"
+#include "attention.hpp"
 #include "attn_q64_loop.inc"
 
 namespace catopt {
@@ -63,39 +63,16 @@ constexpr int QT = 4 * QW;          // queries per workgroup
 constexpr int KVB = 64;   // keys per KV tile
 constexpr float kLazy = 8.0f;
 
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-
 template <int D>
 struct AttnLds {
-  static constexpr int ROW_BYTES = D * 2;
-  static constexpr int CH = D / 8;                  // 16-byte chunks per row
+  static constexpr int ROW_BYTES = AttnRow<D>::BYTES;
+  static constexpr int CH = AttnRow<D>::CH;
   static constexpr int TILE_BYTES = KVB * ROW_BYTES;
   static constexpr int STAGE_BYTES = 2 * TILE_BYTES;  // K then V
   static constexpr int BYTES = 2 * STAGE_BYTES;
   static constexpr int SLOTS = KVB * CH;            // 16-byte slots per tile
   static constexpr int SLOTS_PER_THREAD = SLOTS / NT;
 };
-
-// Byte offset of (key, 16-byte chunk) inside a swizzled tile.
-template <int D>
-__device__ __forceinline__ int tile_off(int key, int chunk) {
-  return key * AttnLds<D>::ROW_BYTES + ((chunk ^ (key & (AttnLds<D>::CH - 1) & 15)) << 4);
-}
-
-// V tiles use their own swizzle.  A transposing read of Vᵀ covers, per
-// 32-lane pass, 4 consecutive keys x 4 adjacent 16-byte chunks; XOR-ing the
-// chunk index with 4 * (the key's position among those 4, per 256-byte bank
-// window) puts the 16 pieces in 16 different bank groups (the key-row
-// swizzle above would put all 4 keys on the same 4 groups).
-template <int D>
-__device__ __forceinline__ int vswz(int key) {
-  constexpr int R = 256 / AttnLds<D>::ROW_BYTES;  // tile rows per 256-byte bank window
-  return 4 * ((key / R) & (4 / R - 1));
-}
-template <int D>
-__device__ __forceinline__ int vtile_off(int key, int chunk) {
-  return key * AttnLds<D>::ROW_BYTES + ((chunk ^ vswz<D>(key)) << 4);
-}
 
 // An empty asm use: the value must be computed before this point, which
 // keeps the compiler from sinking its computation out of an interleaved
@@ -104,11 +81,6 @@ __device__ __forceinline__ void pin(const bf16x8& x) {
   asm volatile("" ::"v"(__builtin_bit_cast(u32x4, x)));
 }
 __device__ __forceinline__ void pin(float x) { asm volatile("" ::"v"(x)); }
-
-__device__ __forceinline__ s16x4 ds_read_tr(const char* lds_base, int byte_off) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) s16x4*)(lds_base + byte_off));
-}
 
 // (head, query tile) of this workgroup in a 1-D grid of nqt x H x B tiles.
 // Workgroups are dealt round robin over the 8 XCDs (linear id L runs on XCD
@@ -787,14 +759,21 @@ bool strides_ok(const int64_t* s) {
 
 using namespace catopt;
 
-extern "C" int32_t catopt_hip_attn_fwd(int32_t dtype, int64_t B, int64_t H, int64_t Tq,
-                                       int64_t Tk, int64_t d, int64_t dv, const void* q,
-                                       const int64_t* q_strides, const void* k,
-                                       const int64_t* k_strides, const void* v,
-                                       const int64_t* v_strides, float scale, int32_t mask_mode,
-                                       int64_t causal_off, const void* mask, int64_t mask_ld,
-                                       int32_t normalize, void* o, const int64_t* o_strides,
-                                       float* m_out, float* l_out, void* stream) {
+extern "C" int64_t catopt_hip_attn_workspace_bytes(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t d) {
+  if (B < 0 || H < 0 || Tq < 0 || Tk < 0 || (d != 64 && d != 128)) return -1;
+  if (B == 0 || H == 0 || Tq == 0 || Tq > kAttnSplitQueries || B > 65535 || H > 65535 || Tk > 0x7fffffffLL) return 0;
+  return attn_split_workspace(B, H, Tq, Tk, d);
+}
+
+extern "C" int32_t catopt_hip_attn_fwd_ws(int32_t dtype, int64_t B, int64_t H, int64_t Tq,
+                                          int64_t Tk, int64_t d, int64_t dv, const void* q,
+                                          const int64_t* q_strides, const void* k,
+                                          const int64_t* k_strides, const void* v,
+                                          const int64_t* v_strides, float scale, int32_t mask_mode,
+                                          int64_t causal_off, const void* mask, int64_t mask_ld,
+                                          int32_t normalize, void* o, const int64_t* o_strides,
+                                          float* m_out, float* l_out, void* workspace,
+                                          int64_t workspace_bytes, void* stream) {
   if (B < 0 || H < 0 || Tq < 0 || Tk < 0) return CATOPT_E_INVAL;
   if (mask_mode < CATOPT_MASK_NONE || mask_mode > CATOPT_MASK_BIAS) return CATOPT_E_INVAL;
   if (normalize < 0 || normalize > 2) return CATOPT_E_INVAL;
@@ -820,6 +799,16 @@ extern "C" int32_t catopt_hip_attn_fwd(int32_t dtype, int64_t B, int64_t H, int6
   auto kp = static_cast<const uint16_t*>(k);
   auto vp = static_cast<const uint16_t*>(v);
   auto op = static_cast<uint16_t*>(o);
+  if (Tq <= kAttnSplitQueries) {
+    AttnArgs a{qp, kp, vp, op, {}, {}, {}, {}, m_out, l_out, B, H, Tq, Tk, causal_off, mask, mask_ld, scale, normalize};
+    for (int i = 0; i < 3; ++i) {
+      a.qs[i] = q_strides[i];
+      a.ks[i] = k_strides[i];
+      a.vs[i] = v_strides[i];
+      a.os[i] = o_strides[i];
+    }
+    return attn_split_launch(a, d, mask_mode, workspace, workspace_bytes, s);
+  }
   if (q64_fits(d, mask_mode, Tk, k_strides, v_strides)) {
     if (mask_mode == CATOPT_MASK_CAUSAL)
       return attn_q64_launch<CATOPT_MASK_CAUSAL>(qp, q_strides, kp, k_strides, vp, v_strides, op, o_strides,
@@ -834,4 +823,17 @@ extern "C" int32_t catopt_hip_attn_fwd(int32_t dtype, int64_t B, int64_t H, int6
   return attn_dispatch_mask<64>(mask_mode, qp, q_strides, kp, k_strides, vp, v_strides, op,
                                 o_strides, m_out, l_out, B, H, Tq, Tk, scale, causal_off, mask,
                                 mask_ld, normalize, s);
+}
+
+extern "C" int32_t catopt_hip_attn_fwd(int32_t dtype, int64_t B, int64_t H, int64_t Tq,
+                                       int64_t Tk, int64_t d, int64_t dv, const void* q,
+                                       const int64_t* q_strides, const void* k,
+                                       const int64_t* k_strides, const void* v,
+                                       const int64_t* v_strides, float scale, int32_t mask_mode,
+                                       int64_t causal_off, const void* mask, int64_t mask_ld,
+                                       int32_t normalize, void* o, const int64_t* o_strides,
+                                       float* m_out, float* l_out, void* stream) {
+  return catopt_hip_attn_fwd_ws(dtype, B, H, Tq, Tk, d, dv, q, q_strides, k, k_strides, v, v_strides, scale,
+                                mask_mode, causal_off, mask, mask_ld, normalize, o, o_strides, m_out, l_out,
+                                nullptr, 0, stream);
 }

@@ -325,10 +325,13 @@ def attention(
     # every operand, and the (B, H, Tq) statistics, advance by whole batches
     for b0 in range(0, B, ATTENTION_MAX_GRID_AXIS):
         nb = min(B - b0, ATTENTION_MAX_GRID_AXIS)
-        st = lib.catopt_hip_attn_fwd(
+        wsb = lib.catopt_hip_attn_workspace_bytes(nb, H, Tq, Tk, d)  # key ranges of a call with few queries
+        ws = _workspace(max(wsb, 0), q.device)
+        st = lib.catopt_hip_attn_fwd_ws(
             L.BF16, nb, H, Tq, Tk, d, dv, _ptr(q[b0:]), qs, _ptr(k[b0:]), ks, _ptr(v[b0:]), vs,
             float(scale), mode, int(causal_off), _ptr(mask_u8), mask_ld, norm, _ptr(o[b0:]), os_,
-            _ptr(m[b0:] if m is not None else None), _ptr(l[b0:] if l is not None else None), _stream(q))
+            _ptr(m[b0:] if m is not None else None), _ptr(l[b0:] if l is not None else None), _ptr(ws), max(wsb, 0),
+            _stream(q))
         L.check("catopt_hip_attn_fwd", st)
     if return_ml:
         return o, m.unsqueeze(-1), l.unsqueeze(-1)

@@ -183,6 +183,26 @@ int32_t catopt_hip_attn_fwd(int32_t dtype, int64_t B, int64_t H, int64_t Tq,
                             float* l_out, void* stream);
 
 /*
+ * catopt_hip_attn_fwd with a workspace: a call with few queries (Tq <= 32)
+ * then splits the keys of each (b, h) over workgroups and combines the
+ * ranges' carriers (the workspace holds them).
+ * catopt_hip_attn_workspace_bytes is the size such a call reads (0: none,
+ * -1: invalid arguments); with less, or NULL, the keys are not split.
+ */
+int64_t catopt_hip_attn_workspace_bytes(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t d);
+int32_t catopt_hip_attn_fwd_ws(int32_t dtype, int64_t B, int64_t H, int64_t Tq,
+                            int64_t Tk, int64_t d, int64_t dv,
+                            const void* q, const int64_t* q_strides,
+                            const void* k, const int64_t* k_strides,
+                            const void* v, const int64_t* v_strides,
+                            float scale, int32_t mask_mode,
+                            int64_t causal_off, const void* mask,
+                            int64_t mask_ld, int32_t normalize, void* o,
+                            const int64_t* o_strides, float* m_out,
+                            float* l_out, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+
+/*
  * Row statistics of an explicit score block for the om element
  * (_om_elem, torch_bridge.py:1974-1981; _batched_elem, om_lower.py:
  * 462-472): for each row r of s [rows, cols] (fp32 or bf16, row stride lds)
