@@ -279,6 +279,10 @@ extern "C" int32_t catopt_hip_linear_ws(int32_t dtype, int64_t M, int64_t N, int
     return launch_skinny(epilogue, static_cast<const float*>(x), ldx, static_cast<const float*>(w), ldw,
                          static_cast<const float*>(bias), static_cast<const float*>(bias2),
                          static_cast<float*>(y), ldy, M, N, K, s);
+  if (dtype == CATOPT_F32 && !paired && gemm_f32_tile_ok(1, M, N, K, x, ldx, 0, false, w, ldw, 0, true))
+    return gemm_f32_tile_launch(epilogue, 1, M, N, K, static_cast<const float*>(x), ldx, 0, false,
+                                static_cast<const float*>(w), ldw, 0, true, static_cast<const float*>(bias),
+                                static_cast<const float*>(bias2), static_cast<float*>(y), ldy, 0, s);
   if (paired) {
     return dtype == CATOPT_BF16 ? dispatch_paired<uint16_t>(epilogue, x, ldx, w, ldw, y, ldy, M, N, K, s)
                                 : dispatch_paired<float>(epilogue, x, ldx, w, ldw, y, ldy, M, N, K, s);
@@ -313,6 +317,11 @@ extern "C" int32_t catopt_hip_matmul(int32_t dtype, int64_t batch, int64_t M, in
       gemm_bf16_nt_fast_ok(M, N, K, A, lda, B, ldb, C, ldc))
     return gemm_bf16_nt_launch(CATOPT_EPI_NONE, M, N, K, A, lda, B, ldb, nullptr, nullptr, C, ldc,
                                batch, strideA, strideB, strideC, nullptr, 0, s);
+  if (dtype == CATOPT_F32 &&
+      gemm_f32_tile_ok(batch, M, N, K, A, lda, strideA, transA != 0, B, ldb, strideB, transB != 0))
+    return gemm_f32_tile_launch(CATOPT_EPI_NONE, batch, M, N, K, static_cast<const float*>(A), lda, strideA,
+                                transA != 0, static_cast<const float*>(B), ldb, strideB, transB != 0, nullptr,
+                                nullptr, static_cast<float*>(C), ldc, strideC, s);
 #define CATOPT_MM(T)                                                                                          \
   if (!transA && !transB) return dispatch_epi<T, false, false>(0, A, lda, strideA, B, ldb, strideB, nullptr, nullptr, C, ldc, strideC, batch, M, N, K, s); \
   if (!transA && transB) return dispatch_epi<T, false, true>(0, A, lda, strideA, B, ldb, strideB, nullptr, nullptr, C, ldc, strideC, batch, M, N, K, s);   \

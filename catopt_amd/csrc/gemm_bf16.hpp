@@ -152,4 +152,11 @@ int32_t gemm_bf16_mid_launch(const GemmMidPlan& plan, int32_t epi, int64_t M, in
                              int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* bias2, void* y,
                              int64_t ldy, void* ws, hipStream_t s);
 
+// fp32 tiles (gemm_f32_tile.hip).  ta: A stored K x M; tb: B stored N x K.
+bool gemm_f32_tile_ok(int64_t batch, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t sA, bool ta,
+                      const void* B, int64_t ldb, int64_t sB, bool tb);
+int32_t gemm_f32_tile_launch(int32_t epi, int64_t batch, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
+                             int64_t sA, bool ta, const float* B, int64_t ldb, int64_t sB, bool tb, const float* bias,
+                             const float* bias2, float* C, int64_t ldc, int64_t sC, hipStream_t s);
+
 }  // namespace catopt
