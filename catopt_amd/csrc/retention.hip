@@ -653,8 +653,15 @@ extern "C" int64_t catopt_hip_retention_workspace_bytes(int64_t B, int64_t H, in
 namespace catopt {
 // fp32 operands (retention_f32.hip): d a multiple of 4 up to 128, any T.
 int32_t retention_f32_launch(int64_t B, int64_t H, int64_t T, int64_t d, const float* q, const float* k,
-                             const float* v, const float* gamma, float scale, float* o, hipStream_t s);
+                             const float* v, const float* gamma, float scale, float* o, void* ws, int64_t ws_bytes,
+                             hipStream_t s);
+int64_t retention_f32_workspace(int64_t B, int64_t H, int64_t T, int64_t d);
 }  // namespace catopt
+
+extern "C" int64_t catopt_hip_retention_f32_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t d) {
+  if (B < 0 || H < 0 || T < 0 || d < 1 || d > 128 || d % 4) return -1;
+  return B == 0 || H == 0 || T == 0 ? 0 : retention_f32_workspace(B, H, T, d);
+}
 
 extern "C" int32_t catopt_hip_retention_fwd(int32_t dtype, int64_t B, int64_t H, int64_t T,
                                             int64_t d, int64_t chunk, const void* q, const void* k,
@@ -662,14 +669,14 @@ extern "C" int32_t catopt_hip_retention_fwd(int32_t dtype, int64_t B, int64_t H,
                                             void* workspace, int64_t workspace_bytes,
                                             void* stream) {
   if (B < 0 || H < 0 || T < 0 || workspace_bytes < 0) return CATOPT_E_INVAL;
-  if (dtype == CATOPT_F32) {  // no workspace: the state stays in registers
+  if (dtype == CATOPT_F32) {  // without a workspace one segment per head
     if (d < 1 || d > 128 || d % 4 || chunk != CH) return CATOPT_E_UNSUPPORTED;
     if (B == 0 || H == 0 || T == 0) return CATOPT_OK;
     if (!q || !k || !v || !gamma || !o) return CATOPT_E_INVAL;
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o)) return CATOPT_E_INVAL;
     return retention_f32_launch(B, H, T, d, static_cast<const float*>(q), static_cast<const float*>(k),
-                                static_cast<const float*>(v), gamma, scale, static_cast<float*>(o),
-                                static_cast<hipStream_t>(stream));
+                                static_cast<const float*>(v), gamma, scale, static_cast<float*>(o), workspace,
+                                workspace_bytes, static_cast<hipStream_t>(stream));
   }
   if (dtype != CATOPT_BF16 || !dims_ok(d, d) || chunk != CH) return CATOPT_E_UNSUPPORTED;
   if (B == 0 || H == 0 || T == 0) return CATOPT_OK;

@@ -3,19 +3,34 @@
 //
 //   o[t] = scale · Σ_{s ≤ t} γ^(t−s) (q[t]·k[s]) v[s]
 //
-// in chunks of C = 64 steps: for chunk n with carried state S (d × dv),
+// in chunks of C = 32 steps: for chunk n with carried state S (d × d),
 //   o_n = scale · ( (q_n k_nᵀ ⊙ D) v_n + diag(γ^a) q_n S ),   D[a, b] = γ^(a−b) (a ≥ b)
 //   S  ← γ^C S + k_nᵀ diag(γ^(C−b)) v_n
 // which is the bf16 kernel's algebra with every operand, product and the
 // state in fp32 (no rounding to bf16 anywhere).
 //
-// Work split.  A workgroup owns one head and a slice of 32 value columns and
-// runs every chunk in order.  Wave w owns q/k columns [32w, 32w + 32): its
-// share of the score q kᵀ, of the inter-chunk term q S and of the state
-// update only ever touches those columns, and all three are linear in them,
-// so each wave produces a partial output of the chunk's 64 x 32 block; the
-// four partials are summed through LDS once per chunk (double-buffered, one
-// barrier per chunk).  The state tile S[32w.., slice] stays in registers.
+// Work split.  The fp32 MFMA bounds it (64 cycles for 32 x 32 x 2), so the
+// split computes nothing twice and puts a wave on every SIMD.  Each head's
+// chunks are cut into P segments; retention_f32<STATE> folds each segment
+// but the last into its state from zero, and retention_f32<OUT> starts each
+// segment from the fold of those before it and emits the outputs.  In a
+// workgroup wave w owns value columns 32w .. 32w + 31 and the state tiles
+// S[:, 32w..]; the 32 x 32 scores of a chunk are split over the waves by q/k
+// columns and their partial sums meet in LDS.  160 MFMAs per wave and chunk
+// at d = 128.  (With a workgroup per 32 value columns and all of a head's
+// chunks in order, each slice recomputed the scores and each wave the whole
+// P v.)  Measured, that kernel and this one: 32 heads x 2048 steps x 128
+// 253 / 103 us, 64 x 8192 x 128 1011 / 600, 32 x 2048 x 64 221 / 45.  A product
+// takes 38-40 ns here (27 at 2.4 GHz; without the loads the 64 x 8192 output
+// pass still takes 409 of 471 us).  With MFMA accumulators in VGPRs
+// (-amdgpu-mfma-vgpr-form) d = 128 is 5% faster and d = 64 16-25% slower: two
+// waves then fit a SIMD and both of a workgroup's may land on one.
+//
+// The q, k and v rows of a chunk go global->LDS directly, one chunk ahead.
+// LDS rows are XOR-swizzled by a permutation of the row's low four bits that
+// keeps both reads free of bank conflicts: 16-byte reads along a row by 32
+// lanes on 32 rows, and 4-byte reads of 32 columns of rows j and j + 4 by the
+// two lane halves.
 //
 // Operand layouts (32x32x2 f32 MFMA: lane l gives A row l%32 and B column
 // l%32 at k index l/32; the accumulator of lane l holds column l%32, rows
@@ -26,231 +41,354 @@
 //   * the state accumulator S[dd, c] (lane: column c, register t: row dd)
 //     is the B operand of the inter term O = Q S;
 //   * the score accumulator Pᵀ[j, i] (lane: query i, register t: key j) is
-//     the A operand of O += P V;
-//   * q and k are loaded so that register t of lane (row, g) holds column
-//     acc_row(t, g) of the wave's 32 columns (four 16-byte loads per tile).
-// v and the key columns of the state update (kᵀ) are read with lanes along
-// a row (128-byte coalesced words).  Loads go through buffer resources over
-// the head's rows: rows past T read zeros; columns past d are given an
-// out-of-range offset and read zeros too.
+//     the A operand of O += P V.
+// Loads go through buffer resources over the head's rows: rows past T and
+// columns past d read zeros, and stores there are dropped.
 #include "common.hpp"
 
 namespace catopt {
 namespace {
 
-constexpr int kC = 64;          // chunk length (steps)
-constexpr int kNT = 256;        // 4 waves
-constexpr int kSlice = 32;      // value columns per workgroup
-constexpr uint32_t kOOB = 0x80000000u;  // a buffer offset past every range: loads 0
+constexpr int kC = 32;                  // chunk length (steps)
+constexpr uint32_t kOOB = 0x80000000u;  // a buffer offset past every range: loads 0, stores nothing
+constexpr int64_t kMaxSeg = 16;
 
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float4 ld4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
-}
-
-__device__ __forceinline__ float ld1(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
-}
-
-// Byte offset of column `col` in a row, or kOOB past the row's width d.  It
-// is added to row offsets below 2^31, so a past-the-width column stays out of
-// range; computed once per lane (and kept opaque) so that no load carries a
-// select the compiler could split into branches around the load.
-__device__ __forceinline__ uint32_t col_bytes(int col, int d) {
-  uint32_t c = col < d ? (uint32_t)col * 4u : kOOB;
-  asm volatile("" : "+v"(c));
-  return c;
-}
-
-// Row-tile operand of q or k: reg[4u + e] = X[row0 + l32][dd0 + 8u + 4g + e]
-// with vrow[u] = l32·d·4 + col_bytes(dd0 + 8u + 4g) and soff = row0·d·4.
-__device__ __forceinline__ void load_rows(__amdgpu_buffer_rsrc_t r, const uint32_t (&vrow)[4], uint32_t soff,
-                                          float (&reg)[16]) {
+// N steps of one or two products with `read` behind them.  With one wave per
+// SIMD an LDS read right before its use is waited out, so every stream of
+// products carries the reads of the next one; and a product that adds to the
+// result of the one before it waits for it, so streams alternate between two
+// accumulators.
+template <int N, typename Product, typename Read>
+__device__ __forceinline__ void stream(Product product, Read read) {
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const float4 x = ld4(r, vrow[u], soff);
-    reg[4 * u + 0] = x.x;
-    reg[4 * u + 1] = x.y;
-    reg[4 * u + 2] = x.z;
-    reg[4 * u + 3] = x.w;
+  for (int x = 0; x < N; ++x) {
+    product(x);
+    read(x);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// Column operand: reg[t] = X[row0 + acc_row(t, g)][col] with
-// vcol = 4g·d·4 + col_bytes(col) and soff = row0·d·4; the rest of the row
-// index, 8(t/4) + t%4, goes into the scalar offset.
-__device__ __forceinline__ void load_cols(__amdgpu_buffer_rsrc_t r, uint32_t vcol, uint32_t soff, int d,
-                                          float (&reg)[16]) {
-#pragma unroll
-  for (int t = 0; t < 16; ++t) reg[t] = ld1(r, vcol, soff + (uint32_t)((8 * (t >> 2) + (t & 3)) * d * 4));
-}
+// ND tiles of 32 columns (d <= 32 ND) and as many waves.
+template <int ND>
+struct Ret {
+  static constexpr int NT = 64 * ND, ROW = 128 * ND;        // threads; bytes of an LDS row
+  static constexpr int CH = 8 * ND;                         // 16-byte chunks of a row
+  static constexpr int MAT = kC * ROW;                      // one matrix of a chunk
+  static constexpr int LOADS = MAT / 1024 / ND;             // 1 KB loads per wave and matrix
+  static constexpr int64_t STATE = 1024LL * ND * ND;        // floats
+  static_assert(CH >= 16, "the swizzle permutes 16 chunks");
+};
 
-__global__ __launch_bounds__(kNT) void retention_f32(const float* __restrict__ q, const float* __restrict__ k,
-                                                     const float* __restrict__ v, const float* __restrict__ gamma,
-                                                     float scale, float* __restrict__ o, int H, int T, int d,
-                                                     int nslice, int remap_rows) {
-  extern __shared__ __attribute__((aligned(16))) float red[];  // [2][4][64][32] partial outputs
-  // XCD-aware order: the hardware deals workgroups to the 8 XCDs round-robin;
-  // remapping keeps consecutive logical ids (a head's slices, which read the
-  // same q and k) on one XCD's L2
-  int bid = blockIdx.x;
-  if (remap_rows > 0) bid = (bid & 7) * remap_rows + (bid >> 3);
-  const int slice = bid % nslice;
-  const int64_t bh = bid / nslice;
+// The swizzle of row r: its low four bits with bits 2 and 3 traded.
+__device__ __forceinline__ int row_swz(int r) { return (r & 3) | ((r & 4) << 1) | ((r & 8) >> 1); }
+
+// Chunks [first, ...) of segment seg.
+__host__ __device__ inline int64_t seg_first(int64_t nch, int64_t seg, int64_t P) { return nch * seg / P; }
+
+template <int ND, bool OUT>
+__global__ __launch_bounds__(64 * ND, 1) void retention_f32(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+    const float* __restrict__ gamma, float scale, float* __restrict__ o, float* __restrict__ pieces, int H, int T,
+    int d, int P) {
+  using L = Ret<ND>;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  constexpr int NMAT = OUT ? 3 : 2, STAGE = NMAT * L::MAT;  // (q,) k, v
+  const int nseg = OUT ? P : P - 1;
+  const int64_t bh = blockIdx.x / nseg;
+  const int seg = blockIdx.x % nseg;
   const int h = (int)(bh % H);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int l32 = lane & 31, g = lane >> 5;
-  const int dd0 = 32 * w;            // this wave's q/k columns
-  const int c0 = kSlice * slice;     // this workgroup's value columns
-  const int nact = (d + 31) / 32;    // waves holding q/k columns
-  const bool active = dd0 < d;
+  const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t base = bh * (int64_t)T * d;
-  const int bytes = T * d * 4;
-  const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)(q + base), (short)0, bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)(k + base), (short)0, bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)(v + base), (short)0, bytes, 0x00020000);
-  float* oh = o + base;
+  const uint32_t bytes = (uint32_t)T * (uint32_t)d * 4u;
+  const u32x4 rq = make_rsrc(q + base, bytes), rk = make_rsrc(k + base, bytes), rv = make_rsrc(v + base, bytes);
+  const int nch = (T + kC - 1) / kC;
+  const int c0 = (int)seg_first(nch, seg, P), c1 = (int)seg_first(nch, seg + 1, P);
 
   // decay factors of this lane, fixed over the chunks (exp2 domain)
   const float gam = gamma[h];
   const float lg = log2f(fabsf(gam));
   const bool neg = gam < 0.f;
-  float rowf[2][16], diagf[16], offf[16], wv[2][16];
+  float rowf[16], diagf[16], wv[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int ar = acc_row(r, g);
-    rowf[0][r] = pow_k(lg, neg, ar);                             // γ^a, a = row in chunk
-    rowf[1][r] = pow_k(lg, neg, 32 + ar);
-    diagf[r] = ar <= l32 ? pow_k(lg, neg, l32 - ar) : 0.f;        // D on diagonal tiles
-    offf[r] = pow_k(lg, neg, 32 + l32 - ar);                      // D on the lower tile
-    wv[0][r] = pow_k(lg, neg, kC - ar);                           // γ^(C − b)
-    wv[1][r] = pow_k(lg, neg, kC - 32 - ar);
+    rowf[r] = pow_k(lg, neg, ar);                            // γ^a, a = row in chunk
+    diagf[r] = ar <= l32 ? pow_k(lg, neg, l32 - ar) : 0.f;    // D
+    wv[r] = pow_k(lg, neg, kC - ar);                         // γ^(C − b)
   }
   const float gC = pow_k(lg, neg, kC);
 
-  // per-lane parts of the load offsets (bytes); row bases go to soffset
-  uint32_t vrow[4];
+  // this wave's loads of a matrix: 1 KB blocks of 1024 / ROW rows
+  uint32_t off[L::LOADS];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) vrow[u] = (uint32_t)(l32 * d * 4) + col_bytes(dd0 + 8 * u + 4 * g, d);
-  const uint32_t vcol_v = (uint32_t)(4 * g * d * 4) + col_bytes(c0 + l32, d);
-  const uint32_t vcol_k = (uint32_t)(4 * g * d * 4) + col_bytes(dd0 + l32, d);
-  const uint32_t tile_b = 32u * (uint32_t)d * 4u;  // bytes of 32 rows
-
-  f32x16 sacc = {};  // S[dd0 + acc_row(r, g)][c0 + l32]
-  const int nch = (T + kC - 1) / kC;
-  float qr[2][16], kr[2][16];
-  if (active) {
-    load_rows(rq, vrow, 0, qr[0]);
-    load_rows(rq, vrow, tile_b, qr[1]);
-    load_rows(rk, vrow, 0, kr[0]);
-    load_rows(rk, vrow, tile_b, kr[1]);
+  for (int i = 0; i < L::LOADS; ++i) {
+    const int slot = 64 * (L::LOADS * w + i) + lane, row = slot / L::CH, chunk = (slot % L::CH) ^ row_swz(row);
+    off[i] = 4 * chunk < d ? (uint32_t)(row * d + 4 * chunk) * 4u : kOOB;
   }
-  for (int n = 0; n < nch; ++n) {
-    const int t0 = n * kC;
-    const uint32_t sb = (uint32_t)t0 * (uint32_t)d * 4u;  // the chunk's first row
-    float* buf = red + (n & 1) * (4 * kC * kSlice);
-    if (active) {
-      float vr[2][16], kc[2][16];
-      load_cols(rv, vcol_v, sb, d, vr[0]);
-      load_cols(rv, vcol_v, sb + tile_b, d, vr[1]);
-      load_cols(rk, vcol_k, sb, d, kc[0]);
-      load_cols(rk, vcol_k, sb + tile_b, d, kc[1]);
-
-      // inter-chunk term, then the per-row decay γ^a
-      f32x16 oacc[2] = {{}, {}};
+  const uint32_t lds0 = lds_u32(lds);
+  auto issue = [&](int n, int stage) {
+    const uint32_t sb = (uint32_t)n * (uint32_t)(kC * d * 4);  // the chunk's first row
+    const uint32_t dst = lds0 + stage * STAGE + L::LOADS * w * 1024;
 #pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        oacc[0] = mfma_f32(qr[0][t], sacc[t], oacc[0]);
-        oacc[1] = mfma_f32(qr[1][t], sacc[t], oacc[1]);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        oacc[0][r] *= rowf[0][r];
-        oacc[1][r] *= rowf[1][r];
-      }
-      // scores Pᵀ[j, i] over this wave's columns: tiles (jt, it) = (0,0), (0,1), (1,1)
-      f32x16 p00 = {}, p01 = {}, p11 = {};
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        p00 = mfma_f32(kr[0][t], qr[0][t], p00);
-        p01 = mfma_f32(kr[0][t], qr[1][t], p01);
-        p11 = mfma_f32(kr[1][t], qr[1][t], p11);
-      }
-      // the next chunk's q and k rows (their registers are free from here)
-      if (n + 1 < nch) {
-        const uint32_t nb = sb + 2u * tile_b;
-        load_rows(rq, vrow, nb, qr[0]);
-        load_rows(rq, vrow, nb + tile_b, qr[1]);
-        load_rows(rk, vrow, nb, kr[0]);
-        load_rows(rk, vrow, nb + tile_b, kr[1]);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        p00[r] *= diagf[r];
-        p11[r] *= diagf[r];
-        p01[r] *= offf[r];
-      }
-      // intra-chunk term O += P V (query tile 0 sees key tile 0, tile 1 both)
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        oacc[0] = mfma_f32(p00[t], vr[0][t], oacc[0]);
-        oacc[1] = mfma_f32(p01[t], vr[0][t], oacc[1]);
-        oacc[1] = mfma_f32(p11[t], vr[1][t], oacc[1]);
-      }
-      // state update S ← γ^C S + kᵀ diag(γ^(C−b)) v over this wave's rows
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sacc[r] *= gC;
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        sacc = mfma_f32(kc[0][t], wv[0][t] * vr[0][t], sacc);
-        sacc = mfma_f32(kc[1][t], wv[1][t] * vr[1][t], sacc);
-      }
-      float* mine = buf + w * (kC * kSlice);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        mine[acc_row(r, g) * kSlice + l32] = oacc[0][r];
-        mine[(32 + acc_row(r, g)) * kSlice + l32] = oacc[1][r];
-      }
+    for (int i = 0; i < L::LOADS; ++i) {
+      // a column past d keeps its out-of-range offset (row offsets stay below 2^31)
+      const uint32_t src = off[i] + sb;
+      if (OUT) dma_buf(rq, src, dst + 2 * L::MAT + i * 1024);
+      dma_buf(rk, src, dst + i * 1024);
+      dma_buf(rv, src, dst + L::MAT + i * 1024);
     }
-    __syncthreads();
-    // wave w sums and stores rows 8w .. 8w + 7 of each 32-row half
-    const int col = c0 + l32;
+  };
+  // X[l32][32 tile + 8 u + 4 g + e], e = 0 .. 3: inner index acc_row(4 u + e, g) of the tile
+  auto row4 = [&](const char* X, int tile, int u) {
+    return *reinterpret_cast<const f32x4*>(X + l32 * L::ROW + (((8 * tile + 2 * u + g) ^ row_swz(l32)) << 4));
+  };
+  // X[acc_row(t, g)][32 tile + l32]
+  auto col1 = [&](const char* X, int tile, int t) {
+    const int j = acc_row(t, g);
+    return *reinterpret_cast<const float*>(X + j * L::ROW + (((8 * tile + (l32 >> 2)) ^ row_swz(j)) << 4) +
+                                           4 * (l32 & 3));
+  };
+
+  if (c0 < c1) issue(c0, 0);
+  f32x16 S[ND];  // S[32 tile + acc_row(r, g)][32 w + l32]
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+  for (int t = 0; t < ND; ++t)
 #pragma unroll
-      for (int it = 0; it < 2; ++it) {
-        const int i = 32 * it + 8 * w + 4 * g + e;
-        float s = 0.f;
+    for (int r = 0; r < 16; ++r) S[t][r] = 0.f;
+  // a state piece in memory: 16 bytes per lane, lanes contiguous
+  auto piece = [&](int64_t s) { return pieces + (bh * (P - 1) + s) * L::STATE + (w * ND * 4 * 64 + lane) * 4; };
+  if (OUT) {  // 64 KB per segment before this one (ND = 4): about 2 us each, bound by one CU's load rate
+    for (int s = 0; s < seg; ++s) {
+      const float f = pow_k(lg, neg, kC * (int)(seg_first(nch, s + 1, P) - seg_first(nch, s, P)));
+      const float* src = piece(s);
 #pragma unroll
-        for (int x = 0; x < 4; ++x) {  // partials of waves past nact were not written: selected out
-          const float px = buf[x * (kC * kSlice) + i * kSlice + l32];
-          s += x < nact ? px : 0.f;
+      for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(src + (4 * t + u) * 256);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) S[t][4 * u + e] = __builtin_fmaf(f, S[t][4 * u + e], x[e]);
         }
-        const int row = t0 + i;
-        if (row < T && col < d) oh[(int64_t)row * d + col] = scale * s;
-      }
     }
   }
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(o + base, (short)0, (int)bytes, 0x00020000);
+  const uint32_t ocol = 32 * w + l32 < d ? (uint32_t)(32 * w + l32 + 4 * g * d) * 4u : kOOB;
+  float* part = reinterpret_cast<float*>(lds + 2 * STAGE);
+  __builtin_amdgcn_s_waitcnt(0);  // the first chunk: no stores behind its loads yet
+
+  for (int n = c0; n < c1; ++n) {
+    const int stage = (n - c0) & 1;
+    // chunk n has landed (its loads are older than the 16 stores of the
+    // chunk before), and every wave is done with the other half and with the
+    // partial scores
+    __builtin_amdgcn_s_waitcnt(OUT ? ((16 & 15) | (7 << 4) | ((16 >> 4) << 14)) : 0);
+    __syncthreads();
+    if (n + 1 < c1) issue(n + 1, stage ^ 1);
+    const char* Ks = lds + stage * STAGE;
+    const char* Vs = Ks + L::MAT;
+    const char* Qs = Vs + L::MAT;
+    float vr[16], kc[ND][16];
+    f32x16 oacc;
+    if (OUT) {
+      f32x16 p, o2;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[r] = oacc[r] = o2[r] = 0.f;
+      f32x4 kf[4], qw[4], qf[ND][4], ps[ND][4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        kf[u] = row4(Ks, w, u);
+        qw[u] = row4(Qs, w, u);
+        qf[0][u] = row4(Qs, 0, u);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // scores Pᵀ[j, i] over this wave's q/k columns, and the inter-chunk
+      // term's first tile
+      stream<16>(
+          [&](int x) {
+            p = mfma_f32(kf[x >> 2][x & 3], qw[x >> 2][x & 3], p);
+            oacc = mfma_f32(qf[0][x >> 2][x & 3], S[0][x], oacc);
+          },
+          [&](int x) {
+            if (x % 4 == 0) qf[1][x >> 2] = row4(Qs, 1, x >> 2);
+            if (ND == 4 && x % 4 == 2) qf[ND - 2][x >> 2] = row4(Qs, ND - 2, x >> 2);
+          });
+      // the partial scores go to LDS; the inter-chunk term's next tiles
+      auto put = [&](int u) {
+        *reinterpret_cast<f32x4*>(part + ((4 * w + u) * 64 + lane) * 4) =
+            f32x4{p[4 * u], p[4 * u + 1], p[4 * u + 2], p[4 * u + 3]};
+      };
+      if (ND == 4) {
+        stream<16>(
+            [&](int x) {
+              oacc = mfma_f32(qf[1][x >> 2][x & 3], S[1][x], oacc);
+              o2 = mfma_f32(qf[ND - 2][x >> 2][x & 3], S[ND - 2][x], o2);
+            },
+            [&](int x) {
+              if (x % 4 == 0) qf[ND - 1][x >> 2] = row4(Qs, ND - 1, x >> 2);
+              if (x % 4 == 3) put(x >> 2);
+            });
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) put(u);
+      }
+      __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (3 << 14));  // lgkmcnt 0
+      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+      // the last tile, while the partial scores come back from all waves
+      stream<8>(
+          [&](int x) {
+            const int y = 2 * x;
+            oacc = mfma_f32(qf[ND - 1][y >> 2][y & 3], S[ND - 1][y], oacc);
+            o2 = mfma_f32(qf[ND - 1][y >> 2][(y & 3) + 1], S[ND - 1][y + 1], o2);
+          },
+          [&](int x) {
+#pragma unroll
+            for (int y = 2 * x; y < 2 * x + 2; ++y) {
+              vr[y] = col1(Vs, w, y);
+              if (y < 4 * ND) ps[y >> 2][y & 3] = *reinterpret_cast<const f32x4*>(part + (y * 64 + lane) * 4);
+            }
+          });
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        oacc[r] = (oacc[r] + o2[r]) * rowf[r];  // the per-row decay γ^a
+        o2[r] = 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int y = 1; y < ND; ++y) ps[0][u] += ps[y][u];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ps[0][u][e] *= diagf[4 * u + e];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // intra-chunk term O += P V
+      stream<8>(
+          [&](int x) {
+            const int y = 2 * x;
+            oacc = mfma_f32(ps[0][y >> 2][y & 3], vr[y], oacc);
+            o2 = mfma_f32(ps[0][y >> 2][(y & 3) + 1], vr[y + 1], o2);
+          },
+          [&](int x) {
+#pragma unroll
+            for (int y = 2 * x; y < 2 * x + 2; ++y) {
+              kc[0][y] = col1(Ks, 0, y);
+              kc[1][y] = col1(Ks, 1, y);
+            }
+          });
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[r] += o2[r];
+    } else {
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        vr[x] = col1(Vs, w, x);
+        kc[0][x] = col1(Ks, 0, x);
+        kc[1][x] = col1(Ks, 1, x);
+      }
+    }
+    // state update S ← γ^C S + kᵀ diag(γ^(C−b)) v (not read again past the last chunk)
+    if (!OUT || n + 1 < c1) {
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        vr[x] *= wv[x];
+        S[0][x] *= gC;
+        S[1][x] *= gC;
+      }
+#pragma unroll
+      for (int t = 0; t < ND; t += 2) {
+        __builtin_amdgcn_sched_barrier(0);
+        stream<16>(
+            [&](int x) {
+              S[t] = mfma_f32(kc[t][x], vr[x], S[t]);
+              S[t + 1] = mfma_f32(kc[t + 1][x], vr[x], S[t + 1]);
+            },
+            [&](int x) {
+#pragma unroll
+              for (int y = t + 2; y < t + 4 && y < ND; ++y) {
+                kc[y][x] = col1(Ks, y, x);
+                S[y][x] *= gC;
+              }
+            });
+      }
+    }
+    if (OUT) {
+      const uint32_t sb = (uint32_t)n * (uint32_t)(kC * d * 4);
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, scale * oacc[r]), ro,
+                                              (int)(ocol + sb + (uint32_t)((8 * (r >> 2) + (r & 3)) * d * 4)), 0, 0);
+    }
+  }
+  if (!OUT) {
+    float* dst = piece(seg);
+#pragma unroll
+    for (int t = 0; t < ND; ++t)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        *reinterpret_cast<f32x4*>(dst + (4 * t + u) * 256) =
+            f32x4{S[t][4 * u], S[t][4 * u + 1], S[t][4 * u + 2], S[t][4 * u + 3]};
+  }
+}
+
+// Segments per head: one workgroup per CU (two at ND = 2, whose LDS is half),
+// at least two chunks each; past 16 the fold of the start state costs what
+// the shorter segments give.
+int64_t n_segments(int64_t BH, int64_t T, int64_t d) {
+  const int64_t slots = d > 64 ? 256 : 512, nch = (T + kC - 1) / kC;
+  int64_t P = BH > 0 ? slots / BH : 1;
+  if (P > kMaxSeg) P = kMaxSeg;
+  if (P > nch / 2) P = nch / 2;
+  return P < 1 ? 1 : P;
+}
+
+template <int ND>
+int32_t launch(int64_t BH, int64_t H, int64_t T, int64_t d, const float* q, const float* k, const float* v,
+               const float* gamma, float scale, float* o, float* ws, int64_t P, hipStream_t s) {
+  using L = Ret<ND>;
+  constexpr int LDS_STATE = 4 * L::MAT, LDS_OUT = 6 * L::MAT + ND * 4096;
+  static bool attr_done = false;  // idempotent; benign race (same value written)
+  if (!attr_done) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&retention_f32<ND, true>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_OUT);
+    if (e != hipSuccess) return set_hip_error(e);
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&retention_f32<ND, false>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS_STATE);
+    if (e != hipSuccess) return set_hip_error(e);
+    attr_done = true;
+  }
+  if (P > 1) {
+    retention_f32<ND, false><<<dim3((uint32_t)(BH * (P - 1))), dim3(L::NT), LDS_STATE, s>>>(
+        q, k, v, gamma, scale, o, ws, (int)H, (int)T, (int)d, (int)P);
+    CATOPT_LAUNCH_CHECK();
+  }
+  retention_f32<ND, true><<<dim3((uint32_t)(BH * P)), dim3(L::NT), LDS_OUT, s>>>(q, k, v, gamma, scale, o, ws, (int)H,
+                                                                                (int)T, (int)d, (int)P);
+  CATOPT_LAUNCH_CHECK();
+  return CATOPT_OK;
 }
 
 }  // namespace
 
+int64_t retention_f32_workspace(int64_t B, int64_t H, int64_t T, int64_t d) {
+  const int64_t P = n_segments(B * H, T, d);
+  return B * H * (P - 1) * (d > 64 ? Ret<4>::STATE : Ret<2>::STATE) * (int64_t)sizeof(float);
+}
+
 int32_t retention_f32_launch(int64_t B, int64_t H, int64_t T, int64_t d, const float* q, const float* k,
-                             const float* v, const float* gamma, float scale, float* o, hipStream_t s) {
+                             const float* v, const float* gamma, float scale, float* o, void* ws, int64_t ws_bytes,
+                             hipStream_t s) {
   if (d < 1 || d > 128 || d % 4) return CATOPT_E_UNSUPPORTED;
-  if (T * d * 4 + (int64_t)kC * d * 4 > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;  // 32-bit buffer offsets
-  const int nslice = (int)((d + kSlice - 1) / kSlice);
-  const int64_t grid = B * H * nslice;
-  if (grid > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;
-  const int remap_rows = grid % 8 == 0 ? (int)(grid / 8) : 0;
-  const size_t lds = 2 * 4 * kC * kSlice * sizeof(float);
-  retention_f32<<<dim3((uint32_t)grid), dim3(kNT), lds, s>>>(q, k, v, gamma, scale, o, (int)H, (int)T, (int)d,
-                                                             nslice, remap_rows);
-  CATOPT_LAUNCH_CHECK();
-  return CATOPT_OK;
+  if (T * d * 4 + 2 * (int64_t)kC * d * 4 > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;  // 32-bit buffer offsets
+  if (B * H * kMaxSeg > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;
+  int64_t P = n_segments(B * H, T, d);
+  if (P > 1 && (!ws || !aligned16(ws) || ws_bytes < retention_f32_workspace(B, H, T, d))) P = 1;
+  float* pieces = static_cast<float*>(ws);
+  return d > 64 ? launch<4>(B * H, H, T, d, q, k, v, gamma, scale, o, pieces, P, s)
+                : launch<2>(B * H, H, T, d, q, k, v, gamma, scale, o, pieces, P, s);
 }
 
 }  // namespace catopt

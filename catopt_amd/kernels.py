@@ -397,8 +397,8 @@ def retention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gamma: torch.Te
     ``v (B,H,T,dv)``, all bf16, fp32 or fp16 (widened to fp32), ``dk, dv <=
     128``.  The kernels
     read a head dim ``d`` (a multiple of 8 for bf16, of 4 for fp32) and any
-    ``T`` in place: columns past ``d`` and rows past ``T`` of the 64-step
-    chunks load as zeros and are never stored.  When ``dk`` and ``dv``
+    ``T`` in place: columns past ``d`` and rows past ``T`` of the last chunk
+    load as zeros and are never stored.  When ``dk`` and ``dv``
     differ, or are not such multiples, the narrower operands run zero-padded
     to the common width (zero columns leave q·k unchanged and add zero output
     columns, dropped).  fp32 operands compute in fp32 throughout."""
@@ -430,11 +430,12 @@ def retention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gamma: torch.Te
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     o = torch.empty_like(v)
     dt = L.F32 if q.dtype == torch.float32 else L.BF16
-    wsb = 0  # the fp32 kernel keeps its state in registers and takes no workspace
     if dt == L.BF16:
         wsb = lib.catopt_hip_retention_workspace_bytes(B, H, T, d, RETENTION_CHUNK)
-        if wsb < 0:
-            raise ValueError("retention workspace query rejected the shape")
+    else:
+        wsb = lib.catopt_hip_retention_f32_workspace_bytes(B, H, T, d)
+    if wsb < 0:
+        raise ValueError("retention workspace query rejected the shape")
     ws = _workspace(wsb, q.device)
     st = lib.catopt_hip_retention_fwd(dt, B, H, T, d, RETENTION_CHUNK, _ptr(q), _ptr(k),
                                       _ptr(v), _ptr(g), float(scale), _ptr(o), _ptr(ws), wsb,

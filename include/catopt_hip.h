@@ -245,13 +245,16 @@ int32_t catopt_hip_om_compose(int64_t rows, int64_t dv, const float* m1,
  * d a multiple of 8 up to 128) or CATOPT_F32 (operands, products and state
  * in fp32; d a multiple of 4 up to 128); gamma: [H] fp32; chunk ∈ {64}; any
  * T (rows past T of the last chunk read as zeros and are not stored).
- * Workspace (bf16 only; the fp32 kernel takes none and ignores it):
- * catopt_hip_retention_workspace_bytes(...) bytes, any contents — the
- * per-segment start-state pieces when T is split into segments over the
- * current device's CUs, 0 when one segment per head fills the device
- * (without a device, the bound for the most segments any device takes).
- * -1 for an unsupported d / chunk.
+ * Workspace (bf16): catopt_hip_retention_workspace_bytes(...) bytes, any
+ * contents — the per-segment start-state pieces when T is split into
+ * segments over the current device's CUs, 0 when one segment per head fills
+ * the device (without a device, the bound for the most segments any device
+ * takes).  -1 for an unsupported d / chunk.  fp32 calls use up to
+ * catopt_hip_retention_f32_workspace_bytes(...) bytes the same way; with
+ * less, or NULL, each head runs as one segment.
  */
+int64_t catopt_hip_retention_f32_workspace_bytes(int64_t B, int64_t H, int64_t T,
+                                                 int64_t d);
 int64_t catopt_hip_retention_workspace_bytes(int64_t B, int64_t H, int64_t T,
                                              int64_t d, int64_t chunk);
 int32_t catopt_hip_retention_fwd(int32_t dtype, int64_t B, int64_t H,
