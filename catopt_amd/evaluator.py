@@ -421,7 +421,9 @@ class HipIRModule(nn.Module):
 
     def _eval(self, t: Any, env: dict, x: Any, memo: dict) -> Any:
         """Evaluate a subterm (used by the planned executors for their leaves)."""
-        ops = self._bindings()
+        # a leaf (an input, a Param, a constant) reads no binding: the table
+        # of 258, resolved per call, cost 2 us for each of a layer's operands
+        ops = self._bindings() if is_op(t) else None
         return eval_term(t, env, self._param_map, ops, memo, default=x)
 
     def _eval_fast(self, t: Any, env: dict, x: Any) -> Any:

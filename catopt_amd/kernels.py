@@ -227,6 +227,9 @@ def _bhtd(t: torch.Tensor) -> tuple[torch.Tensor, list[int]]:
 
 ATTENTION_MAX_HEAD_DIM = 128
 
+#: Largest query count of the kernel that splits the keys (a workspace call).
+ATTENTION_FEW_QUERIES = 32
+
 
 #: Largest batch and head extents of one ``catopt_hip_attn_fwd`` launch
 #: (CATOPT_E_UNSUPPORTED beyond them).  :func:`attention` splits a larger
@@ -323,15 +326,22 @@ def attention(
     norm = (2 if empty_rows == "zero" else 1) if normalize else 0
     # one launch per run of at most ATTENTION_MAX_GRID_AXIS batch entries:
     # every operand, and the (B, H, Tq) statistics, advance by whole batches
+    few = Tq <= ATTENTION_FEW_QUERIES
     for b0 in range(0, B, ATTENTION_MAX_GRID_AXIS):
         nb = min(B - b0, ATTENTION_MAX_GRID_AXIS)
-        wsb = lib.catopt_hip_attn_workspace_bytes(nb, H, Tq, Tk, d)  # key ranges of a call with few queries
-        ws = _workspace(max(wsb, 0), q.device)
-        st = lib.catopt_hip_attn_fwd_ws(
-            L.BF16, nb, H, Tq, Tk, d, dv, _ptr(q[b0:]), qs, _ptr(k[b0:]), ks, _ptr(v[b0:]), vs,
-            float(scale), mode, int(causal_off), _ptr(mask_u8), mask_ld, norm, _ptr(o[b0:]), os_,
-            _ptr(m[b0:] if m is not None else None), _ptr(l[b0:] if l is not None else None), _ptr(ws), max(wsb, 0),
-            _stream(q))
+        part = (q, k, v, o, m, l)
+        if nb != B:
+            part = tuple(None if t is None else t[b0:] for t in part)
+        qp, kp, vp, op, mp, lp = (None if t is None else t.data_ptr() for t in part)
+        args = (L.BF16, nb, H, Tq, Tk, d, dv, qp, qs, kp, ks, vp, vs, float(scale), mode, int(causal_off),
+                _ptr(mask_u8), mask_ld, norm, op, os_, mp, lp)
+        # a call with few queries splits its keys over a workspace
+        wsb = lib.catopt_hip_attn_workspace_bytes(nb, H, Tq, Tk, d) if few else 0
+        if wsb > 0:
+            ws = _workspace(wsb, q.device)
+            st = lib.catopt_hip_attn_fwd_ws(*args, _ptr(ws), wsb, _stream(q))
+        else:
+            st = lib.catopt_hip_attn_fwd(*args, _stream(q))
         L.check("catopt_hip_attn_fwd", st)
     if return_ml:
         return o, m.unsqueeze(-1), l.unsqueeze(-1)
