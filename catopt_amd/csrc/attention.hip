@@ -679,7 +679,7 @@ template <int MASK>
 int32_t attn_q64_launch(const uint16_t* q, const int64_t* qs, const uint16_t* k, const int64_t* ks,
                         const uint16_t* v, const int64_t* vs, uint16_t* o, const int64_t* os, float* m_out,
                         float* l_out, int64_t B, int64_t H, int64_t Tq, int64_t Tk, float scale,
-                        int64_t causal_off, int normalize, hipStream_t s) {
+                        int64_t causal_off, int normalize, int paired, hipStream_t s) {
   static bool attr_done = false;
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_q64_kernel<MASK>),
@@ -688,8 +688,6 @@ int32_t attn_q64_launch(const uint16_t* q, const int64_t* qs, const uint16_t* k,
     attr_done = true;
   }
   const int64_t nqt = (Tq + QT64 - 1) / QT64;
-  // an even number of query tiles goes two to a workgroup
-  const int paired = nqt % 2 == 0 ? 1 : 0;
   const int64_t nblk = (paired ? nqt / 2 : nqt) * H * B;
   if (nblk > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;
   attn_q64_kernel<MASK><<<dim3((uint32_t)nblk), dim3(NT), LDS64, s>>>(
@@ -705,6 +703,30 @@ bool q64_fits(int64_t d, int32_t mode, int64_t Tk, const int64_t* ks, const int6
   if (d != 128 || (mode != CATOPT_MASK_NONE && mode != CATOPT_MASK_CAUSAL)) return false;
   if (Tk <= 0 || Tk % 64 != 0) return false;
   return ((Tk - 1) * ks[2] + 128) * 2 < 0x7fffffffLL && ((Tk - 1) * vs[2] + 128) * 2 < 0x7fffffffLL;
+}
+
+// Whether the 64-query kernel pays for `heads` heads of Tq queries, and whether
+// its query tiles then go two to a workgroup (an even number of them).  It
+// is 10-16% faster than the 32-query kernel on full rounds of workgroups, one
+// to a CU, but its unit of work is four times as large (two of the other's
+// workgroups, of half the queries, share a CU), so a part-filled round costs
+// more than that.  Measured at d = 128, causal / full, in us, the 32-query
+// kernel first: n = 32 tiles (1 x 16 heads, T = 512) 16 against 35 / 39; n =
+// 128 (1 x 16, 2048) 46 against 56 / 47 against 56; n = 256 (1 x 32, 2048) 63
+// against 58 / 76 against 68, where pairs would leave half the CUs idle (72 /
+// 119); n = 416 (13 x 8, 1024) 54 against 49; n = 512 (4 x 32, 1024) 59
+// against 53; n = 768 (6 x 32, 1024) 81 against 95; n = 1536 (6 x 32, 2048)
+// 259 against 245.  Up to two query tiles the prologue and epilogue take
+// what the faster tiles give (8 x 32, T = 512: 41 against 45).
+bool q64_pays(int64_t heads, int64_t Tq, int* paired) {
+  constexpr int64_t kCus = 256;
+  const int64_t nqt = (Tq + QT64 - 1) / QT64, n = nqt * heads;
+  *paired = 0;
+  if (nqt <= 2 || n <= kCus * 11 / 16) return false;
+  if (n <= kCus) return true;
+  *paired = nqt % 2 == 0;
+  const int64_t wgs = *paired ? n / 2 : n, slots = (wgs + kCus - 1) / kCus * kCus;
+  return wgs * 100 >= slots * (slots == kCus ? 70 : 85);
 }
 
 template <int D, int MASK>
@@ -809,12 +831,14 @@ extern "C" int32_t catopt_hip_attn_fwd_ws(int32_t dtype, int64_t B, int64_t H, i
     }
     return attn_split_launch(a, d, mask_mode, workspace, workspace_bytes, s);
   }
-  if (q64_fits(d, mask_mode, Tk, k_strides, v_strides)) {
+  int paired = 0;
+  if (q64_fits(d, mask_mode, Tk, k_strides, v_strides) && q64_pays(B * H, Tq, &paired)) {
     if (mask_mode == CATOPT_MASK_CAUSAL)
       return attn_q64_launch<CATOPT_MASK_CAUSAL>(qp, q_strides, kp, k_strides, vp, v_strides, op, o_strides,
-                                                 m_out, l_out, B, H, Tq, Tk, scale, causal_off, normalize, s);
+                                                 m_out, l_out, B, H, Tq, Tk, scale, causal_off, normalize, paired,
+                                                 s);
     return attn_q64_launch<CATOPT_MASK_NONE>(qp, q_strides, kp, k_strides, vp, v_strides, op, o_strides, m_out,
-                                             l_out, B, H, Tq, Tk, scale, causal_off, normalize, s);
+                                             l_out, B, H, Tq, Tk, scale, causal_off, normalize, paired, s);
   }
   if (d == 128)
     return attn_dispatch_mask<128>(mask_mode, qp, q_strides, kp, k_strides, vp, v_strides, op,
