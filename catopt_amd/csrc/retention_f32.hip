@@ -383,7 +383,7 @@ int32_t retention_f32_launch(int64_t B, int64_t H, int64_t T, int64_t d, const f
                              hipStream_t s) {
   if (d < 1 || d > 128 || d % 4) return CATOPT_E_UNSUPPORTED;
   if (T * d * 4 + 2 * (int64_t)kC * d * 4 > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;  // 32-bit buffer offsets
-  if (B * H * kMaxSeg > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;
+  if (B * H > 0x7fffffffLL) return CATOPT_E_UNSUPPORTED;  // more segments than one: B H <= 256
   int64_t P = n_segments(B * H, T, d);
   if (P > 1 && (!ws || !aligned16(ws) || ws_bytes < retention_f32_workspace(B, H, T, d))) P = 1;
   float* pieces = static_cast<float*>(ws);
