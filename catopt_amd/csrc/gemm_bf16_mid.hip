@@ -14,9 +14,11 @@
 // 64 through a ring of STAGES LDS slots: both operands' rows go global->LDS
 // directly (whole 128-byte lines, rows XOR-swizzled so that a fragment read
 // hits 16 distinct 16-byte bank groups), STAGES - 1 stages ahead, with one
-// barrier per stage.  What bounds the loop is bytes in flight: a two-slot
-// ring of 128 x 128 tiles, two workgroups per CU, had 64 KB per CU in flight
-// and ran at half this kernel's rate.
+// barrier per stage.  What bounds the loop is the stage's load latency and
+// bytes: 0.63 us per 128 x 256 x 64 stage with the operands cached, 0.80 us
+// with W from HBM, where the MFMAs take 0.4 us.  A two-slot ring of 128 x 128
+// tiles, two workgroups per CU, needed 0.83 us for the same work and cached
+// operands.
 #include "common.hpp"
 #include "gemm_bf16.hpp"
 
@@ -137,7 +139,8 @@ __global__ __launch_bounds__(2 * BN, 2) void gemm_bf16_mid(MidArgs g) {
   // One half stage: the products of half h with the reads of the next half and
   // some loads among them, one memory instruction between two MFMAs.  Issued in
   // a block, the reads and loads of all waves queue up in front of the first
-  // product (19% slower at 128 x 256).
+  // product: 64 rows x 5504 -> 2048 without K ranges took 72 us for 55 with W
+  // cached, and the same time with W from HBM.
   constexpr int NMEM = G::FN + G::FM, NLOAD = G::XL + G::WL, NLOAD_A = NLOAD / 2;
   auto half = [&](int h, int rslot, int rh, int T, int lslot, int l0, int l1) {
     constexpr int NM = G::FN * G::FM;
