@@ -21,8 +21,10 @@
 //                    every range split where it crosses a segment start);
 //                    reads k and v once more, writes one 64 KB fp32 state
 //                    per piece;
+//   retention_fold   (more than 8 segments) the state at each segment start
+//                    from the pieces before it, in place;
 //   retention_out    one workgroup per (b, h, segment): sums its start state
-//                    from the pieces, then walks the segment's chunks, so q,
+//                    from the pieces (or reads the folded one), then walks the segment's chunks, so q,
 //                    k, v and o cross HBM once there and each chunk's q, k, v
 //                    tiles cross global->LDS once per head.
 // With P = 1 (enough heads to fill the chip) retention_out alone runs, from
@@ -80,7 +82,8 @@ constexpr int STAGE_A = 2 * TILE;
 constexpr int LDS_A = NSTAGE_A * STAGE_A;
 static_assert(LDS_A <= 160 * 1024, "retention_state LDS");
 constexpr int WFLOATS = HD * HD;       // one state piece: 128 x 128 fp32
-constexpr int MAXSEG = 8;
+constexpr int MAXSEG = 32;
+constexpr int SUMSEG = 8;              // past these, retention_fold makes the start states
 constexpr int MAXPIECE = 2 * MAXSEG;
 constexpr uint32_t kOOB = 0x80000000u;  // a buffer offset past every range: loads 0, stores dropped
 
@@ -538,8 +541,9 @@ __global__ __launch_bounds__(NT, 1) void retention_out(
     for (int r = 0; r < 16; ++r) S[t][r] = 0.f;
   if (s > 0) {
     const float* ph = pieces + (int64_t)bh * 2 * plan.nseg * WFLOATS;
+    const bool folded = plan.nseg > SUMSEG;  // the piece that ends at c0 is the state there
     for (int p = 0; p < 2 * plan.nseg; ++p) {
-      if (plan.r0[p] >= plan.r1[p] || plan.r1[p] > c0) continue;
+      if (plan.r0[p] >= plan.r1[p] || plan.r1[p] > c0 || (folded && plan.r1[p] < c0)) continue;
       const float fct = pow_k(lg, neg, (c0 - plan.r1[p]) * CH);
       const f32x4* src = reinterpret_cast<const f32x4*>(ph + (int64_t)p * WFLOATS);
 #pragma unroll
@@ -568,11 +572,51 @@ __global__ __launch_bounds__(NT, 1) void retention_out(
     out_segment<3>(lds, qh, kh, vh, oh, T, dk, dv, scale, lg, neg, c0, c1, S, L, w, tid);
 }
 
-// Segments per head: about one workgroup per CU in all, at least two chunks
-// per segment, at most MAXSEG.
-int n_segments(int64_t BH, int64_t nch, int n_cu) {
-  int64_t p = (n_cu + BH - 1) / BH;
-  if (p > MAXSEG) p = MAXSEG;
+// With more than SUMSEG segments: each piece that ends at a segment start
+// becomes the state there, S_p = γ^(length) S_(p-1) + piece, in place.  A
+// thread owns four floats of a head's state and walks the pieces in order,
+// eight loads in flight.  Summed in retention_out instead, the last of 32
+// segments would read 62 pieces of 64 KB through one CU (about 35 us).
+__global__ __launch_bounds__(NT) void retention_fold(const float* __restrict__ gamma, int H, SegPlan plan,
+                                                     float* pieces) {
+  constexpr int F4 = WFLOATS / 4, BATCH = 8;
+  const int bh = blockIdx.x, n = 2 * plan.nseg;
+  f32x4* base = reinterpret_cast<f32x4*>(pieces) + (int64_t)bh * n * F4 + blockIdx.y * NT + threadIdx.x;
+  const float gam = gamma[bh % H];
+  const float lg = __log2f(fabsf(gam));
+  const bool neg = gam < 0.f;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  int s = 1;  // the next segment start
+  for (int p0 = 0; p0 < n; p0 += BATCH) {
+    f32x4 x[BATCH];
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) x[i] = base[(int64_t)min(p0 + i, n - 1) * F4];
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      const int p = p0 + i;
+      if (p >= n || plan.r0[p] >= plan.r1[p]) continue;  // an empty piece holds anything
+      acc = pow_k(lg, neg, (plan.r1[p] - plan.r0[p]) * CH) * acc + x[i];
+      if (plan.r1[p] == plan.seg[s]) {
+        base[(int64_t)p * F4] = acc;
+        ++s;
+      }
+    }
+  }
+}
+
+// Segments per head.  A workgroup's LDS fills a CU, so one round of them is
+// the most that helps: 48 heads took 171 us in 288 workgroups and 115 in 240
+// (T = 8192, d = 128).  At least two chunks a segment; more than SUMSEG only
+// where that leaves four chunks each and saves enough of the chain to pay for
+// retention_fold: 4 heads 66 -> 43 us at T = 8192 and 41 -> 34 at 4096, 16
+// heads 67 -> 52 (d = 64) and 45 -> 43, but 31 -> 35 with two chunks (T = 2048).
+int n_segments(int64_t BH, int64_t nch, int n_cu, int most) {
+  int64_t p = n_cu / BH;
+  if (p > SUMSEG) {
+    if (p > most) p = most;
+    if (p > nch / 4) p = nch / 4;
+    if (p < SUMSEG + 4) p = SUMSEG;
+  }
   if (p > nch / 2) p = nch / 2;
   return p < 1 ? 1 : (int)p;
 }
@@ -640,12 +684,12 @@ extern "C" int64_t catopt_hip_retention_workspace_bytes(int64_t B, int64_t H, in
   if (B < 0 || H < 0 || T < 0 || !dims_ok(d, d) || chunk != CH) return -1;
   const int64_t BH = B * H, nch = (T + CH - 1) / CH;
   if (BH == 0 || nch == 0) return 0;
-  // the current device's segment count; without a device, the most any
-  // device can take (the bound on segments alone)
+  // the current device's segment count; without a device, SUMSEG at most
+  // (a call given less than more segments need runs on SUMSEG)
   int n_cu = 0, dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    n_cu = 0x3fffffff;
-  const int P = n_segments(BH, nch, n_cu);
+    n_cu = 0;
+  const int P = n_cu > 0 ? n_segments(BH, nch, n_cu, MAXSEG) : n_segments(BH, nch, 0x3fffffff, SUMSEG);
   if (P == 1) return 0;
   return BH * 2 * P * WFLOATS * (int64_t)sizeof(float);  // two state pieces per range
 }
@@ -684,16 +728,18 @@ extern "C" int32_t catopt_hip_retention_fwd(int32_t dtype, int64_t B, int64_t H,
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o)) return CATOPT_E_INVAL;
   const int64_t BH = B * H, nch = (T + CH - 1) / CH;
   // 32-bit buffer ranges per chunk, int chunk indices, grid within 2^31
-  if (BH * MAXSEG > 0x7fffffffLL || nch > 0x3fffffffLL) return CATOPT_E_UNSUPPORTED;
+  if (BH * SUMSEG > 0x7fffffffLL || nch > 0x3fffffffLL) return CATOPT_E_UNSUPPORTED;
   int n_cu = 0;
   int32_t st = cu_count_of_current_device(&n_cu);
   if (st != CATOPT_OK) return st;
-  const int P = n_segments(BH, nch, n_cu);
+  const auto need = [&](int P) { return BH * 2 * P * WFLOATS * (int64_t)sizeof(float); };
+  int P = n_segments(BH, nch, n_cu, MAXSEG);
+  if (P > SUMSEG && workspace_bytes < need(P)) P = SUMSEG;
   const SegPlan plan = make_plan(P, nch);
   if (!plan_ok(plan)) return CATOPT_E_UNSUPPORTED;
   if (P > 1) {
     if (!workspace || !aligned16(workspace)) return CATOPT_E_INVAL;
-    if (workspace_bytes < BH * 2 * P * WFLOATS * (int64_t)sizeof(float)) return CATOPT_E_WORKSPACE;
+    if (workspace_bytes < need(P)) return CATOPT_E_WORKSPACE;
   }
   static bool attr_done = false;
   if (!attr_done) {
@@ -713,6 +759,10 @@ extern "C" int32_t catopt_hip_retention_fwd(int32_t dtype, int64_t B, int64_t H,
   if (P > 1) {
     retention_state<<<dim3((uint32_t)(P * BH)), dim3(NT), LDS_A, s>>>(kp, vp, gamma, (int)H, T, (int)d,
                                                                       (int)d, (int)BH, plan, pieces);
+    CATOPT_LAUNCH_CHECK();
+  }
+  if (P > SUMSEG) {
+    retention_fold<<<dim3((uint32_t)BH, WFLOATS / 4 / NT), dim3(NT), 0, s>>>(gamma, (int)H, plan, pieces);
     CATOPT_LAUNCH_CHECK();
   }
   retention_out<<<dim3((uint32_t)(P * BH)), dim3(NT), LDS_C, s>>>(qp, kp, vp, gamma, (int)H, T, (int)d,

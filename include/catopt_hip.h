@@ -248,8 +248,8 @@ int32_t catopt_hip_om_compose(int64_t rows, int64_t dv, const float* m1,
  * Workspace (bf16): catopt_hip_retention_workspace_bytes(...) bytes, any
  * contents — the per-segment start-state pieces when T is split into
  * segments over the current device's CUs, 0 when one segment per head fills
- * the device (without a device, the bound for the most segments any device
- * takes).  -1 for an unsupported d / chunk.  fp32 calls use up to
+ * the device (without a device, the bound for eight segments; a call that
+ * would take more runs on eight when given no more than those need).  -1 for an unsupported d / chunk.  fp32 calls use up to
  * catopt_hip_retention_f32_workspace_bytes(...) bytes the same way; with
  * less, or NULL, each head runs as one segment.
  */
