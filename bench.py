@@ -585,8 +585,8 @@ class C5SSM(Form):
                 "a_t (B,T,D,N) = exp(-softplus(N(0,1))), b_t,c_t (B,T,N), x_t (B,T,D)")
     peak = PEAK["hbm_gbs"]
     work = dom_work = 4.0 * (B * T * D * N + 2 * B * T * N + 2 * B * T * D)
-    dom_name = "ssm_stream_reg<16>"
-    dom_key = "ssm_stream_reg<16>"
+    dom_name = "ssm_segment<16, true, true>"
+    dom_key = "ssm_segment<16, true, true>"
 
     def setup(self, dev):
         import torch

@@ -12,10 +12,10 @@
 //
 // Work split.  A head's state is 128 x 128 fp32, and its chunks are a chain,
 // so a head runs on one workgroup per T-segment: the chunks split into P
-// equal segments (P * B * H about the CU count), and segment s starts from
+// equal segments (P * B * H at most the CU count), and segment s starts from
 //   S_start(s) = sum over chunk ranges R before segment s of γ^((c_s - r1(R)) C) W_R,
 //   W_R = sum_{i in R} γ^((r1 - 1 - i) C) D_i,   D_i = sum_c γ^(C-c) k_ic ⊗ v_ic.
-// Two kernels:
+// Kernels:
 //   retention_state  the W_R of the chunks before the last segment, that
 //                    prefix cut into P equal ranges (one workgroup each,
 //                    every range split where it crosses a segment start);
