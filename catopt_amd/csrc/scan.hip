@@ -299,6 +299,8 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_apply(
 //                 state), reading a, b and x;
 //   EMIT = true   starts each segment from h0 folded through the segments
 //                 before it, and emits y.
+// 8 x 8192 x 2048 x 16: 1790 us a call (5.4 TB/s) where the chunk-parallel
+// schedule, which reads a twice in three launches, took 4300.
 // HBM bounds both, and below two workgroups per CU what bounds a workgroup
 // is the latency of its loads: with loads one stage ahead a stage took 1.66 us
 // (20 GB/s per workgroup).  So everything is loaded two stages ahead: a's
