@@ -96,36 +96,19 @@ __device__ __forceinline__ uint32_t lds_u32(const void* p) {
       reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)p));
 }
 
-// Direct global->LDS load of 16 bytes per lane: lane l's bytes land at LDS
-// byte address lds_wave + 16 l (lds_wave is wave-uniform; it goes to M0).
-// Issued as inline asm: for the builtin form the compiler treats every later
-// transposing LDS read (ds_read_b64_tr_b16) as a possible reader of the load
-// and waits for all loads in flight before it, which serialises a prefetch
-// with the tile being computed.  Callers wait with s_waitcnt vmcnt before
-// the barrier that publishes the loaded stage.
-__device__ __forceinline__ void dma16(const void* gptr, uint32_t lds_wave) {
-  // one wait state between the SALU write of M0 and the LDS-DMA load that
-  // reads it (a hazard the compiler cannot see inside inline asm)
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_wave)
-               : "m0");
-}
-
-// Direct global->LDS load of 4 bytes per lane (lane l's word lands at
-// lds_wave + 4 l), as dma16: inline asm, so the compiler neither waits for it
-// before unrelated LDS accesses nor counts it; callers wait with s_waitcnt
-// vmcnt before the barrier that publishes the data.
-__device__ __forceinline__ void dma4(const void* gptr, uint32_t lds_wave) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gptr), "s"(lds_wave)
-               : "m0");
-}
-
 // One 1 KB global->LDS load through a buffer resource: lane l's 16 bytes at
 // byte `voff` of the buffer land at LDS byte address lds + 16 l (lds is
 // wave-uniform; it goes to M0).  A load past the resource's range returns
 // zeros.  The s_nop is the one wait state the hardware needs between an SALU
 // write of M0 and an LDS-DMA load reading it (the compiler cannot insert it
 // inside inline asm; without it the load can take the previous M0 and land in
-// another load's place).  Inline asm for the reason given at dma16.
+// another load's place).  Issued as inline asm: for the builtin form the
+// compiler treats every later transposing LDS read (ds_read_b64_tr_b16) as a
+// possible reader of the load and waits for all loads in flight before it,
+// which serialises a prefetch with the tile being computed.  The compiler does
+// not count these loads: callers wait with s_waitcnt vmcnt before the barrier
+// that publishes the loaded stage, and such a count covers only operations
+// the compiler cannot move or drop (asm with the "memory" clobber, stores).
 // `lds` goes through readfirstlane: under SGPR pressure the compiler may hold
 // a uniform value in a VGPR, which an "s" operand cannot take.
 __device__ __forceinline__ void dma_buf(u32x4 rsrc, uint32_t voff, uint32_t lds) {

@@ -303,24 +303,23 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_apply(
 // schedule, which reads a twice in three launches, took 4300.
 // HBM bounds both, and below two workgroups per CU what bounds a workgroup
 // is the latency of its loads: with loads one stage ahead a stage took 1.66 us
-// (20 GB/s per workgroup).  So everything is loaded two stages ahead: a's
-// slices for RSU steps go straight into one of three register sets, the
-// small x, b and c streams through LDS (one copy per workgroup, three
-// buffers) by direct loads issued before a's, and y leaves through LDS as
-// whole rows.  The loads have no lane-dependent branch around them, so the
-// waits the compiler derives for a are exact, and the wait at the end of a
-// stage leaves the newest 2 RSU operations in flight across the barrier: it
-// covers the next stage's small streams, which are older than its a.  On
-// gfx9 stores count in vmcnt too, which is why y is not stored step by step
-// under a lane mask.  y's stores are non-temporal (written once, never read
-// back here): 1.5% faster at C5's shape than plain stores.  What y costs
-// beyond that is HBM's turnaround between reads and writes; a plain
-// streaming kernel with the same 16:1 read/write mix pays it as well.  Steps
-// past the last whole stage run unpipelined.
-#ifndef CATOPT_SSM_RSU
-#define CATOPT_SSM_RSU 8
-#endif
-constexpr int RSU = CATOPT_SSM_RSU;  // steps per stage
+// (20 GB/s per workgroup).  So everything is loaded two stages ahead, into
+// one of three register sets: a's slices for RSU steps and this thread's
+// share of the small x, b and c streams.  The share goes to LDS (one copy per
+// workgroup, three buffers) one stage before it is read, and y leaves
+// through LDS as whole rows.  Every load is an ordinary load into registers,
+// so the compiler derives every wait and no result depends on the order in
+// which it places them.  No load has a branch around it: a lane past the end
+// of a small stream repeats another lane's slot.  In two stages of three the
+// derived waits leave the newest two stages in flight.  The loop's back edge
+// joins paths of one, two and three stages, and there the compiler waits for
+// every load, so the run-ahead starts anew with each third stage.
+// y's stores are non-temporal (written once, never read back here): 1.5%
+// faster at C5's shape than plain stores.  What y costs beyond that is
+// HBM's turnaround between reads and writes; a plain streaming kernel with
+// the same 16:1 read/write mix pays it as well.  Steps past the last whole
+// stage run unpipelined.
+constexpr int RSU = 8;  // steps per stage
 
 template <int N>
 struct SsmSmall {
@@ -331,7 +330,14 @@ struct SsmSmall {
   static constexpr int BYTES = 3 * (STAGE + Y_BYTES);
   static constexpr int XPT = (X_SLOTS + kThreads - 1) / kThreads;  // x loads (and y stores) per thread
   static constexpr int VPT = (V_SLOTS + kThreads - 1) / kThreads;  // b and c loads per thread
-  static_assert(X_SLOTS % 64 == 0 && V_SLOTS % 64 == 0, "whole waves per small stream");
+  static_assert(X_SLOTS % 64 == 0, "store_y's guards are wave-uniform");
+};
+
+// One thread's loads of a stage: a's slices, and its slots of x and of b, c.
+template <int N>
+struct SsmStage {
+  f32x4 a[RSU];
+  float x[SsmSmall<N>::XPT], v[SsmSmall<N>::VPT];
 };
 
 // The stages [first, second) of RSU steps that segment seg of P walks (the
@@ -373,45 +379,45 @@ __global__ __launch_bounds__(kThreads, 2) void ssm_segment(
   int xw[L::XPT];
 #pragma unroll
   for (int i = 0; i < L::XPT; ++i) {
-    const int s = i * kThreads + tid, u = s / L::DPW;
+    const int s = (i * kThreads + tid) % L::X_SLOTS, u = s / L::DPW;
     const int cc = (int)(d0 + s % L::DPW < D ? s % L::DPW : D - 1 - d0);
     xo[i] = u * D + d0 + cc;
     xw[i] = u * L::DPW + cc;
   }
+  // and its b and c slots: RSU * N of b, then of c (not emitting, b alone)
+  constexpr int VS = EMIT ? L::V_SLOTS : L::V_SLOTS / 2, VPT = (VS + kThreads - 1) / kThreads;
   const uint32_t ao = (uint32_t)(APS ? (dd - d0) * N + n0 : dd - d0);
 
-  const uint32_t lds0 = lds_u32(lds);
-  // the guards are wave-uniform: every stream is a whole number of waves
-  auto issue_small = [&](int64_t st, int stage) {
-    const uint32_t xb = lds0 + stage * L::STAGE;
+  // stage st into registers, the small streams first (they are used first)
+  auto load = [&](int64_t st, SsmStage<N>& r) {
     const int64_t bt = b * T + st * RSU;
-    const float* xr = x + bt * D;
 #pragma unroll
-    for (int i = 0; i < L::XPT; ++i)
-      if (i * kThreads + wave * 64 < L::X_SLOTS) dma4(xr + xo[i], xb + (i * kThreads + wave * 64) * 4);
-    // b then c, one 4-byte slot per lane: slots [0, RSU*N) of b, then of c
-    // (not emitting, b alone)
+    for (int i = 0; i < L::XPT; ++i) r.x[i] = x[bt * D + xo[i]];
 #pragma unroll
-    for (int i = 0; i < L::VPT; ++i) {
-      const int s = i * kThreads + tid;
-      if (i * kThreads + wave * 64 < (EMIT ? L::V_SLOTS : L::V_SLOTS / 2)) {
-        const bool is_c = s >= RSU * N;
-        dma4((is_c ? c : bx) + bt * N + (is_c ? s - RSU * N : s), xb + (L::X_SLOTS + i * kThreads + wave * 64) * 4);
-      }
+    for (int i = 0; i < VPT; ++i) {
+      const int s = (i * kThreads + tid) % VS;
+      r.v[i] = s < RSU * N ? bx[bt * N + s] : c[bt * N + s - RSU * N];
     }
-  };
-  auto load_a = [&](int64_t st, f32x4* ra) {
-    const float* ar = a + ((b * T + st * RSU) * D + d0) * (APS ? N : 1);
+    const float* ar = a + (bt * D + d0) * (APS ? N : 1);
     const int64_t row = D * (APS ? N : 1);
 #pragma unroll
     for (int u = 0; u < RSU; ++u) {
       if (APS) {
-        ra[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(ar + u * row + ao));
+        r.a[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(ar + u * row + ao));
       } else {
         const float av = (ar + u * row)[ao];
-        ra[u] = f32x4{av, av, av, av};
+        r.a[u] = f32x4{av, av, av, av};
       }
     }
+  };
+  // a stage's small streams into LDS buffer `buf` (a repeated slot: the same
+  // value to the same word)
+  auto put = [&](const SsmStage<N>& r, int buf) {
+    float* xb = reinterpret_cast<float*>(lds + buf * L::STAGE);
+#pragma unroll
+    for (int i = 0; i < L::XPT; ++i) xb[(i * kThreads + tid) % L::X_SLOTS] = r.x[i];
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) xb[L::X_SLOTS + (i * kThreads + tid) % VS] = r.v[i];
   };
 
   f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f}, p = f32x4{1.f, 1.f, 1.f, 1.f};
@@ -424,18 +430,18 @@ __global__ __launch_bounds__(kThreads, 2) void ssm_segment(
     for (int64_t k0 = 0; k0 < seg; k0 += kBatch) {
       f32x4 pk[kBatch], hk[kBatch];
 #pragma unroll
-      for (int i = 0; i < kBatch; ++i)
-        if (k0 + i < seg) {
-          pk[i] = *reinterpret_cast<const f32x4*>(ws_p + (k0 + i) * S + sidx);
-          hk[i] = *reinterpret_cast<const f32x4*>(ws_h + (k0 + i) * S + sidx);
-        }
+      for (int i = 0; i < kBatch; ++i) {  // past the last: that one again, not used (no branch between the loads)
+        const int64_t k = k0 + i < seg ? k0 + i : seg - 1;
+        pk[i] = *reinterpret_cast<const f32x4*>(ws_p + k * S + sidx);
+        hk[i] = *reinterpret_cast<const f32x4*>(ws_h + k * S + sidx);
+      }
 #pragma unroll
       for (int i = 0; i < kBatch; ++i)
         if (k0 + i < seg) h = pk[i] * h + hk[i];
     }
   }
-  auto compute = [&](int stage, const f32x4* ra, char* yb) {
-    const char* xb = lds + stage * L::STAGE;
+  auto compute = [&](int buf, const f32x4* ra, char* yb) {
+    const char* xb = lds + buf * L::STAGE;
     const char* vb = xb + L::X_SLOTS * 4;
     float r[RSU];
 #pragma unroll
@@ -475,35 +481,33 @@ __global__ __launch_bounds__(kThreads, 2) void ssm_segment(
         __builtin_nontemporal_store(*reinterpret_cast<const float*>(yb + xw[i] * 4), yr + xo[i]);
     }
   };
-  // vmcnt <= 2 RSU, lgkmcnt 0
-  auto landed = [&]() {
-    __builtin_amdgcn_s_waitcnt((2 * RSU & 15) | (7 << 4) | ((2 * RSU >> 4) << 14));
-    __syncthreads();
+  auto issue = [&](int64_t st, SsmStage<N>& r) {
+    load(st < st1 ? st : st1 - 1, r);    // past the end: the last stage again, not used
+    __builtin_amdgcn_sched_barrier(0);  // ahead of the products that hide it
   };
-  auto issue = [&](int64_t st, int buf, f32x4* ra) {
-    const int64_t sn = st < st1 ? st : st1 - 1;  // past the end: the last stage again, not read
-    issue_small(sn, buf);
-    load_a(sn, ra);
-  };
-  // stage st from buffer and register set `buf`, stage st + 2 into `ahead`
-  auto step = [&](int64_t st, int buf, const f32x4* cur, int ahead, f32x4* nxt) {
-    issue(st + 2, ahead, nxt);
+  // stage st from register set `cur` and buffer `buf`; stage st + 1's small
+  // streams go to buffer `nbuf`, stage st + 2 into `ahead`.  A buffer is
+  // written two barriers after its last reader's stage began, and read past
+  // the barrier that follows the write.
+  auto step = [&](int64_t st, int buf, const SsmStage<N>& cur, int nbuf, const SsmStage<N>& nxt, SsmStage<N>& ahead) {
+    issue(st + 2, ahead);
     char* yb = lds + 3 * L::STAGE + buf * L::Y_BYTES;
-    compute(buf, cur, yb);
-    landed();
+    compute(buf, cur.a, yb);
+    put(nxt, nbuf);
+    __syncthreads();
     if (EMIT) store_y(st, yb);
   };
-  f32x4 ra0[RSU], ra1[RSU], ra2[RSU];
+  SsmStage<N> r0, r1, r2;
   if (st0 < st1) {
-    issue(st0, 0, ra0);
-    issue(st0 + 1, 1, ra1);
-    landed();
+    issue(st0, r0);
+    issue(st0 + 1, r1);
+    put(r0, 0);
+    __syncthreads();
     for (int64_t st = st0; st < st1; st += 3) {
-      step(st, 0, ra0, 2, ra2);
-      if (st + 1 < st1) step(st + 1, 1, ra1, 0, ra0);
-      if (st + 2 < st1) step(st + 2, 2, ra2, 1, ra1);
+      step(st, 0, r0, 1, r1, r2);
+      if (st + 1 < st1) step(st + 1, 1, r1, 2, r2, r0);
+      if (st + 2 < st1) step(st + 2, 2, r2, 0, r0, r1);
     }
-    __builtin_amdgcn_s_waitcnt(0);  // the loads past the end have landed in LDS
   }
   if (!EMIT) {
     if (!dok) return;

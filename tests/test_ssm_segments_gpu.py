@@ -23,6 +23,9 @@ TOL_F32 = 1e-5
 CASES = [  # B, T, D
     (1, 5, 64), (1, 16, 130), (2, 31, 70), (1, 32, 64), (1, 257, 64),
     (3, 300, 100), (1, 1000, 1), (2, 259, 513), (90, 40, 16), (1, 40, 5700),
+    # every remainder of the stages over the three register sets: 3, 7 (and 5
+    # above) in one pass, 3, 4 and 5 in each of four segments
+    (90, 24, 16), (90, 56, 16), (60, 96, 16), (60, 128, 16), (60, 163, 16),
 ]
 
 
