@@ -298,7 +298,10 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_apply(
 //   EMIT = false  composes each segment but the last into (prod a, local
 //                 state), reading a, b and x;
 //   EMIT = true   starts each segment from h0 folded through the segments
-//                 before it, and emits y.
+//                 before it, and emits y.  It reads the copy of h0 that the
+//                 first launch left in the workspace: its last segment
+//                 writes h_final, which may be h0's own buffer, while the
+//                 others may not have begun.
 // 8 x 8192 x 2048 x 16: 1790 us a call (5.4 TB/s) where the chunk-parallel
 // schedule, which reads a twice in three launches, took 4300.
 // HBM bounds both, and below two workgroups per CU what bounds a workgroup
@@ -511,6 +514,9 @@ __global__ __launch_bounds__(kThreads, 2) void ssm_segment(
   }
   if (!EMIT) {
     if (!dok) return;
+    // the last segment's place in ws_h is not used: h0's copy
+    if (seg == 0 && h0)
+      *reinterpret_cast<f32x4*>(ws_h + (P - 1) * S + sidx) = *reinterpret_cast<const f32x4*>(h0 + sidx);
     *reinterpret_cast<f32x4*>(ws_p + seg * S + sidx) = p;
     *reinterpret_cast<f32x4*>(ws_h + seg * S + sidx) = h;
     return;
@@ -584,6 +590,7 @@ int32_t ssm_launch(int64_t B, int64_t T, int64_t D, const float* a, const float*
       ssm_segment<N, APS, false><<<dim3((uint32_t)gx, (uint32_t)B, (uint32_t)(P - 1)), dim3(kThreads), 0, s>>>(
           a, bx, c, x, h0, T, D, S, P, ws_p, ws_h, y, hf);
       CATOPT_LAUNCH_CHECK();
+      if (h0) h0 = ws_h + (P - 1) * S;
     }
     ssm_segment<N, APS, true><<<dim3((uint32_t)gx, (uint32_t)B, (uint32_t)P), dim3(kThreads), 0, s>>>(
         a, bx, c, x, h0, T, D, S, P, ws_p, ws_h, y, hf);

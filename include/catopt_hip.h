@@ -287,8 +287,8 @@ int32_t catopt_hip_hbm_read(const void* src, int64_t nbytes, uint32_t* sink,
 
 /* scan schedules (catopt_hip_affd_scan, catopt_hip_ssm_scan) */
 enum catopt_scan_schedule {
-  CATOPT_SCAN_AUTO = 0,       /* streaming when the lanes fill the GPU, else chunk-parallel */
-  CATOPT_SCAN_STREAM = 1,     /* one pass: each lane walks the chunks in order */
+  CATOPT_SCAN_AUTO = 0,       /* one pass when the lanes fill the GPU, else in parallel parts of T */
+  CATOPT_SCAN_STREAM = 1,     /* one pass in time order */
   CATOPT_SCAN_CHUNKED = 2     /* chunk-parallel: local chunk maps, carry over chunks, re-scan */
 };
 
@@ -365,14 +365,20 @@ int32_t catopt_hip_affd_scan_noalloc(int64_t T, int64_t S, const float* a,
  * fp32; a: [B,T,D,N] contiguous (a_per_state = 1) or [B,T,D] broadcast
  * over N (a_per_state = 0); bx, c: [B,T,N]; x, y: [B,T,D]; h0, h_final:
  * [B,D,N] (optional, NULL h0 = 0).  N ∈ {4, 8, 16, 32, 64}; any D.  The
- * n-reduction runs across lanes with DPP/ds_swizzle shuffles.  Chunk table
- * and schedule as for catopt_hip_affd_scan; workspace for the
- * chunk-parallel schedule: catopt_hip_scan_workspace_bytes(B*D*N, n_chunks).
+ * n-reduction runs across lanes with DPP moves.  h_final may be h0's buffer
+ * (the state updated in place); no other output may overlap an input.
+ * Schedules: CATOPT_SCAN_AUTO makes one pass, or where B * D * N leaves
+ * the GPU unfilled cuts T into segments of its own choosing, at most
+ * n_chunks of them (two launches); CATOPT_SCAN_STREAM makes one pass.
+ * Neither reads the table's entries, which must tile [0, T) as for
+ * catopt_hip_affd_scan; CATOPT_SCAN_CHUNKED walks them as that call does.
+ * Workspace, 16-byte aligned, for the segments and for CHUNKED:
+ * catopt_hip_scan_workspace_bytes(B*D*N, n_chunks).
  */
 /*
  * The bytes a catopt_hip_ssm_scan call with these sizes and this schedule
- * reads from its workspace (0 when it streams); -1 for a bad size, N or
- * schedule.
+ * needs as its workspace (0 when it makes one pass); -1 for a bad size, N
+ * or schedule.
  */
 int64_t catopt_hip_ssm_scan_workspace_bytes(int64_t B, int64_t T, int64_t D, int64_t N,
                                             int64_t n_chunks, int32_t schedule);

@@ -50,3 +50,27 @@ def test_ssm_auto(B, T, D, N, aps):
     for ref, out in ((ry, y), (rh, h)):
         rep = oracle.verify_equiv(ref, out.cpu().double().numpy(), rtol=TOL_F32)
         assert rep["passed"], rep
+
+
+@pytest.mark.parametrize("N,B,T,D", [(16, 60, 163, 16), (8, 1, 257, 64), (4, 3, 300, 100), (16, 90, 56, 16)])
+def test_ssm_state_updated_in_place(N, B, T, D):
+    """h_final in h0's own buffer: the same values as in a buffer of its own."""
+    g = torch.Generator(device="cuda:0").manual_seed(N + T)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda:0")  # noqa: E731
+    a, bx, c, x, h0 = r(B, T, D, N).sigmoid_(), r(B, T, N), r(B, T, N), r(B, T, D), r(B, D, N)
+    lib, cs = L.load(), torch.from_numpy(oracle.prefix_chunk_table(T).astype(np.int64)).cuda()
+    wsb = lib.catopt_hip_ssm_scan_workspace_bytes(B, T, D, N, len(cs) - 1, L.SCAN_AUTO)
+    outs = []
+    for in_place in (False, True):
+        ws = torch.full((max(wsb, 16) // 4,), float("nan"), device="cuda:0")
+        h, y = h0.clone(), torch.empty_like(x)
+        hf = h if in_place else torch.empty_like(h0)
+        st = lib.catopt_hip_ssm_scan(B, T, D, N, a.data_ptr(), 1, bx.data_ptr(), c.data_ptr(), x.data_ptr(), h.data_ptr(),
+                                     cs.data_ptr(), len(cs) - 1, L.SCAN_AUTO, y.data_ptr(), hf.data_ptr(), ws.data_ptr(),
+                                     wsb, torch.cuda.current_stream().cuda_stream)
+        assert st == L.OK
+        outs.append((y, hf))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    ry, rh = oracle.ssm_serial(*(t.cpu().double().numpy() for t in (a, bx, c, x, h0)))
+    for ref, out in zip((ry, rh), outs[1]):
+        assert oracle.verify_equiv(ref, out.cpu().double().numpy(), rtol=TOL_F32)["passed"]
