@@ -39,6 +39,7 @@ SIGNATURES: dict[str, tuple] = {
         _i32,
         [_i32, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i32, _p, _i64, _p, _i64, _p],
     ),
+    "catopt_hip_gemm_route": (_i32, [_i32, _i64, _i64, _i64, _i64, _i32, _i32, _i64, _pi64]),
     "catopt_hip_matmul": (
         _i32,
         [_i32, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i32, _p, _i64, _i64, _i32, _p, _i64, _i64, _p],

@@ -79,6 +79,10 @@ __device__ __forceinline__ constexpr int acc_row(int r, int g) {
   return 8 * (r >> 2) + 4 * g + (r & 3);
 }
 
+// Whether a grid dimension of `blocks` workgroups can be launched: HIP takes
+// fewer than 2^32 work-items in it.
+inline bool grid_fits(int64_t blocks, int64_t threads) { return blocks * threads < (1LL << 32); }
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // γ^k for an integer k >= 0 from lg = log2|γ| and neg = (γ < 0), as pow

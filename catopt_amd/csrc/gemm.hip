@@ -256,6 +256,35 @@ extern "C" int64_t catopt_hip_linear_workspace_bytes(int32_t dtype, int64_t M, i
   return gemm_bf16_mid_workspace(gemm_bf16_mid_plan(M, N, K, paired, n_cu, true), M, N, paired);
 }
 
+extern "C" int32_t catopt_hip_gemm_route(int32_t dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
+                                         int32_t epilogue, int32_t n_cu, int64_t workspace_bytes, int64_t* plan) {
+  if (batch < 1 || M < 1 || N < 1 || K < 1 || n_cu < 1 || epilogue < CATOPT_EPI_NONE || epilogue > CATOPT_EPI_GLU)
+    return -1;
+  if (dtype != CATOPT_F32 && dtype != CATOPT_BF16) return -1;
+  if (plan) plan[0] = plan[1] = plan[2] = 0;
+  const bool paired = epilogue == CATOPT_EPI_SILU_MUL || epilogue == CATOPT_EPI_GLU;
+  const void* p = reinterpret_cast<const void*>((uintptr_t)4096);  // any aligned address: none is read
+  if (dtype == CATOPT_BF16) {
+    if (!gemm_bf16_nt_fast_ok(M, N, K, p, K, p, K, p, N)) return CATOPT_ROUTE_GENERAL;
+    const GemmMidPlan g = gemm_bf16_plan(batch, M, N, K, paired, n_cu, workspace_bytes);
+    if (g.shape == GEMM_ROWS) return CATOPT_ROUTE_ROWS;
+    if (g.shape == GEMM_MID_NONE) return CATOPT_ROUTE_LARGE;
+    const int64_t bm = g.shape == GEMM_MID_128x256 ? 128 : 64, bn = g.shape == GEMM_MID_128x256 ? 256 : 128;
+    const int64_t cols = paired ? bn / 2 : bn, tiles = ((M + bm - 1) / bm) * ((N + cols - 1) / cols);
+    if (plan) {
+      plan[0] = g.splits > 1 ? g.direct : tiles;
+      plan[1] = tiles - plan[0];
+      plan[2] = g.splits > 1 ? g.splits : 0;
+    }
+    return g.shape == GEMM_MID_128x256 ? CATOPT_ROUTE_128x256 : CATOPT_ROUTE_64x128;
+  }
+  if (paired) return CATOPT_ROUTE_GENERAL;
+  if (batch == 1 && skinny_ok(M, N, K, p, K, p, K)) return CATOPT_ROUTE_F32_ROWS;
+  return gemm_f32_tile_ok(batch, M, N, K, p, K, batch == 1 ? 0 : M * K, false, p, K, batch == 1 ? 0 : N * K, true)
+             ? CATOPT_ROUTE_F32_TILE
+             : CATOPT_ROUTE_GENERAL;
+}
+
 extern "C" int32_t catopt_hip_linear_ws(int32_t dtype, int64_t M, int64_t N, int64_t K,
                                         const void* x, int64_t ldx, const void* w, int64_t ldw,
                                         const void* bias, const void* bias2, int32_t epilogue,

@@ -394,20 +394,15 @@ int32_t gemm_bf16_nt_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const 
                             const void* bias2, void* y, int64_t ldy, int64_t batch,
                             int64_t sA, int64_t sB, int64_t sC, void* ws, int64_t ws_bytes, hipStream_t s) {
   const bool paired = epi == CATOPT_EPI_SILU_MUL || epi == CATOPT_EPI_GLU;
-  if (batch == 1) {
-    int n_cu = 0;
-    const int32_t st = gemm_cu_count(&n_cu);
-    if (st != CATOPT_OK) return st;
-    GemmMidPlan plan = gemm_bf16_mid_plan(M, N, K, paired, n_cu, ws != nullptr && aligned16(ws));
-    if (gemm_bf16_mid_workspace(plan, M, N, paired) > ws_bytes)
-      plan = gemm_bf16_mid_plan(M, N, K, paired, n_cu, false);
-    if (plan.shape == GEMM_ROWS)
-      return gemm_bf16_rows_launch(epi, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, 1, 0, 0, 0, s);
-    if (plan.shape != GEMM_MID_NONE)
-      return gemm_bf16_mid_launch(plan, epi, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, ws, s);
-  } else if (M <= 64) {
+  int n_cu = 0;
+  const int32_t st = gemm_cu_count(&n_cu);
+  if (st != CATOPT_OK) return st;
+  const GemmMidPlan plan =
+      gemm_bf16_plan(batch, M, N, K, paired, n_cu, ws != nullptr && aligned16(ws) && ws_bytes > 0 ? ws_bytes : 0);
+  if (plan.shape == GEMM_ROWS)
     return gemm_bf16_rows_launch(epi, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, batch, sA, sB, sC, s);
-  }
+  if (plan.shape != GEMM_MID_NONE)
+    return gemm_bf16_mid_launch(plan, epi, M, N, K, x, ldx, w, ldw, bias, bias2, y, ldy, ws, s);
   auto A = static_cast<const uint16_t*>(x);
   auto B = static_cast<const uint16_t*>(w);
   auto b1 = static_cast<const uint16_t*>(bias);

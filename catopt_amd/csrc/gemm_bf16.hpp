@@ -132,7 +132,8 @@ int32_t gemm_bf16_nt_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const 
                             int64_t strideA, int64_t strideB, int64_t strideC, void* ws,
                             int64_t ws_bytes, hipStream_t s);
 
-// Few rows, M <= 64 (gemm_bf16_skinny.hip).
+// Few rows, M <= 64 (gemm_bf16_skinny.hip), where its grid can be launched.
+bool gemm_bf16_rows_ok(int64_t M, int64_t N);
 int32_t gemm_bf16_rows_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
                               const void* w, int64_t ldw, const void* bias, const void* bias2, void* y,
                               int64_t ldy, int64_t batch, int64_t sX, int64_t sW, int64_t sC,
@@ -147,6 +148,8 @@ struct GemmMidPlan {
   int shape, direct, round, splits;
 };
 GemmMidPlan gemm_bf16_mid_plan(int64_t M, int64_t N, int64_t K, bool paired, int n_cu, bool ws);
+// The plan of a launch: a batch, and `ws_bytes` of workspace (0: none).
+GemmMidPlan gemm_bf16_plan(int64_t batch, int64_t M, int64_t N, int64_t K, bool paired, int n_cu, int64_t ws_bytes);
 int64_t gemm_bf16_mid_workspace(const GemmMidPlan& p, int64_t M, int64_t N, bool paired);
 int32_t gemm_bf16_mid_launch(const GemmMidPlan& plan, int32_t epi, int64_t M, int64_t N, int64_t K, const void* x,
                              int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* bias2, void* y,

@@ -302,7 +302,7 @@ GemmMidPlan gemm_bf16_mid_plan(int64_t M, int64_t N, int64_t K, bool paired, int
   // Few rows: gemm_bf16_rows reads W once at HBM rate, but X once per 16
   // columns.  17 rows: 8.2 against 9.3 us at 2752 -> 1024, 29.7 against 22.9
   // at 11008 -> 4096; 64 rows, without K ranges: 61 against 89 us.
-  if (M <= 16 || (M <= 48 && wrows * K <= 8 << 20) || (M <= 64 && !ws)) {
+  if (gemm_bf16_rows_ok(M, N) && (M <= 16 || (M <= 48 && wrows * K <= 8 << 20) || !ws)) {
     best.shape = GEMM_ROWS;
     return best;
   }
@@ -316,7 +316,6 @@ GemmMidPlan gemm_bf16_mid_plan(int64_t M, int64_t N, int64_t K, bool paired, int
     return (double)(((M + bm - 1) / bm) * ((N + cols - 1) / cols));
   };
   double cost = rounds(tiles(256, 256), n_cu, kst, 1.05, 1.52) + 4.3;
-  if (tiles(64, 128) > 0x3fffffff) return best;
   const struct {
     int shape, bm, bn, per_cu;
     double lo, hi, launch, reduce, mb_per_us;
@@ -324,6 +323,7 @@ GemmMidPlan gemm_bf16_mid_plan(int64_t M, int64_t N, int64_t K, bool paired, int
                  {GEMM_MID_64x128, 64, 128, 2, 0.27, 0.60, 4.1, 3.0, 2.9}};
   for (const auto& sh : shapes) {
     const double t = tiles(sh.bm, sh.bn), slots = (double)n_cu * sh.per_cu;
+    if (!grid_fits((int64_t)t + n_cu, 2 * sh.bn)) continue;  // at most n_cu workgroups for split tiles
     auto consider = [&](double c, int64_t direct, int64_t splits) {
       if (c < 0.98 * cost) {
         cost = c;
@@ -344,6 +344,15 @@ GemmMidPlan gemm_bf16_mid_plan(int64_t M, int64_t N, int64_t K, bool paired, int
              direct, splits);
   }
   return best;
+}
+
+GemmMidPlan gemm_bf16_plan(int64_t batch, int64_t M, int64_t N, int64_t K, bool paired, int n_cu, int64_t ws_bytes) {
+  if (batch != 1) return GemmMidPlan{gemm_bf16_rows_ok(M, N) ? GEMM_ROWS : GEMM_MID_NONE, 0, n_cu, 1};
+  if (ws_bytes > 0) {
+    const GemmMidPlan p = gemm_bf16_mid_plan(M, N, K, paired, n_cu, true);
+    if (gemm_bf16_mid_workspace(p, M, N, paired) <= ws_bytes) return p;
+  }
+  return gemm_bf16_mid_plan(M, N, K, paired, n_cu, false);
 }
 
 int64_t gemm_bf16_mid_workspace(const GemmMidPlan& p, int64_t M, int64_t N, bool paired) {

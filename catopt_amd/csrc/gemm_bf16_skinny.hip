@@ -165,6 +165,10 @@ int32_t launch_rows(const uint16_t* X, int64_t ldx, const uint16_t* W, int64_t l
 
 }  // namespace
 
+bool gemm_bf16_rows_ok(int64_t M, int64_t N) {
+  return M <= 64 && grid_fits((N + SKN - 1) / SKN, 64 * rows_waves((int)((M + 15) / 16)));
+}
+
 int32_t gemm_bf16_rows_launch(int32_t epi, int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
                               const void* w, int64_t ldw, const void* bias, const void* bias2, void* y,
                               int64_t ldy, int64_t batch, int64_t sX, int64_t sW, int64_t sC,

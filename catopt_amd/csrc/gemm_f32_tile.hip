@@ -184,7 +184,7 @@ bool operand_ok(const void* p, int64_t ld, int64_t stride, int64_t rows, int64_t
 bool gemm_f32_tile_ok(int64_t batch, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t sA, bool ta,
                       const void* B, int64_t ldb, int64_t sB, bool tb) {
   const int64_t tiles = ((M + FT - 1) / FT) * ((N + FT - 1) / FT);
-  return tiles <= 0x7fffffffLL && batch <= 65535 && M < 0x40000000LL && N < 0x40000000LL && K < 0x40000000LL &&
+  return grid_fits(tiles, FNT) && batch <= 65535 && M < 0x40000000LL && N < 0x40000000LL && K < 0x40000000LL &&
          operand_ok(A, lda, sA, M, K, ta) && operand_ok(B, ldb, sB, N, K, !tb);
 }
 

@@ -130,6 +130,29 @@ int32_t catopt_hip_linear_ws(int32_t dtype, int64_t M, int64_t N, int64_t K,
                              void* stream);
 
 /*
+ * The kernel a product of contiguous, 16-byte aligned operands runs on, for
+ * tests and tools (host only, no device needed): catopt_hip_linear_ws at
+ * batch = 1, catopt_hip_matmul with transB at batch > 1, on a device of n_cu
+ * compute units and with workspace_bytes of workspace.  plan (NULL, or 3
+ * values) receives the tiles done whole, the tiles whose K is split, and the
+ * K ranges of each of those (0, 0, 0 outside the middle tiles).  Returns a
+ * catopt_gemm_route, or -1 for invalid arguments.
+ */
+enum catopt_gemm_route {
+  CATOPT_ROUTE_GENERAL = 0,    /* element-wise loads, any layout */
+  CATOPT_ROUTE_ROWS = 1,       /* bf16, few rows: 16 weight rows per workgroup */
+  CATOPT_ROUTE_128x256 = 2,    /* bf16, middle tiles */
+  CATOPT_ROUTE_64x128 = 3,
+  CATOPT_ROUTE_LARGE = 4,      /* bf16, persistent 256 x 256 tiles */
+  CATOPT_ROUTE_F32_ROWS = 5,   /* fp32, few rows: 16 x 16 tiles */
+  CATOPT_ROUTE_F32_TILE = 6    /* fp32, 64 x 64 tiles */
+};
+int32_t catopt_hip_gemm_route(int32_t dtype, int64_t batch, int64_t M,
+                              int64_t N, int64_t K, int32_t epilogue,
+                              int32_t n_cu, int64_t workspace_bytes,
+                              int64_t* plan);
+
+/*
  * Batched matrix product with optional transposes:
  *   C[b] = op(A[b]) · op(B[b]),  op(X) = X or Xᵀ,  C[b] is M × N.
  * A[b] is M×K (transA=0, row stride lda) or K×M (transA=1); B[b] is K×N

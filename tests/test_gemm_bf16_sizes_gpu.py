@@ -114,3 +114,14 @@ def test_batched_few_rows(nb, M, N, Kd):
     y = K.matmul(a, b.transpose(-1, -2))
     for i in range(nb):
         _check(y[i], *_reference(a[i], b[i], L.EPI_NONE, None, None))
+
+
+def test_linear_more_weight_rows_than_the_few_row_grid_takes():
+    # 2^32 work-items at one workgroup of 1024 per 16 rows: other tiles run it
+    N, Kd = 67_108_880, 8
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn((1, Kd), generator=g, device=DEV).to(BF)
+    w = torch.empty((N, Kd), dtype=BF, device=DEV)
+    w.normal_(generator=g)
+    y = K.linear(x, w)
+    _check(y, *_reference(x, w, L.EPI_NONE, None, None))
