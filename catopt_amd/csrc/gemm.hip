@@ -253,7 +253,7 @@ extern "C" int64_t catopt_hip_linear_workspace_bytes(int32_t dtype, int64_t M, i
   int n_cu = 0;
   if (gemm_cu_count(&n_cu) != CATOPT_OK) return 0;  // no device: nothing will be launched
   const bool paired = epilogue == CATOPT_EPI_SILU_MUL || epilogue == CATOPT_EPI_GLU;
-  return gemm_bf16_mid_workspace(gemm_bf16_mid_plan(M, N, K, paired, n_cu, true), M, N, paired);
+  return gemm_bf16_mid_workspace(gemm_bf16_plan(1, M, N, K, paired, n_cu, INT64_MAX), M, N, paired);
 }
 
 extern "C" int32_t catopt_hip_gemm_route(int32_t dtype, int64_t batch, int64_t M, int64_t N, int64_t K,

@@ -147,8 +147,7 @@ enum { GEMM_MID_NONE = 0, GEMM_ROWS, GEMM_MID_128x256, GEMM_MID_64x128 };
 struct GemmMidPlan {
   int shape, direct, round, splits;
 };
-GemmMidPlan gemm_bf16_mid_plan(int64_t M, int64_t N, int64_t K, bool paired, int n_cu, bool ws);
-// The plan of a launch: a batch, and `ws_bytes` of workspace (0: none).
+// The plan of a launch with `ws_bytes` of workspace (0: none).
 GemmMidPlan gemm_bf16_plan(int64_t batch, int64_t M, int64_t N, int64_t K, bool paired, int n_cu, int64_t ws_bytes);
 int64_t gemm_bf16_mid_workspace(const GemmMidPlan& p, int64_t M, int64_t N, bool paired);
 int32_t gemm_bf16_mid_launch(const GemmMidPlan& plan, int32_t epi, int64_t M, int64_t N, int64_t K, const void* x,

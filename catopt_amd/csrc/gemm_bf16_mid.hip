@@ -287,73 +287,112 @@ int32_t run_shape(const MidArgs& a, int shape, hipStream_t s) {
 
 }  // namespace
 
-// Which kernel runs a bf16 NT product, by the time each would take: a whole
-// number of rounds of workgroups, each round K / 64 stages long, at a stage
-// time that grows with the share of the chip at work (the clock falls and the
-// L2s fill), plus the launch and, with K ranges, the second launch and the
-// partial sums' bytes.  The stage times (us, an idle chip and a full one) are
-// fits to 160 measured sizes (N, K from 1024 to 11008, both plain and gated,
-// 20 to 6000 rows), where the kernel chosen here was within 1.3% of the best
-// one on average and 15% at worst; the chip's clock moves them together, so
-// the choice does not depend on it.  Without a workspace no tile is split.
-GemmMidPlan gemm_bf16_mid_plan(int64_t M, int64_t N, int64_t K, bool paired, int n_cu, bool ws) {
+// Which kernel runs a bf16 NT product (or a batch of them), by the time each
+// would take in us.  The constants are fits to 1242 single and 1765 batched
+// sizes, plain and gated, 1 to 4096 rows, N from 32 to 131072, K from 64 to
+// 11008, weights from memory (profiles/gemm_bf16_routes.md): the kernel chosen
+// here is within 1.6% of the best one on average, 0.7% without a workspace and
+// 0.3% in a batch, and at most 8% slower than the large tiles.  Before, few rows
+// took the few-rows kernel whatever N and the batch were: 64 rows x 4096 ->
+// 131072 630 us for 258 on the large tiles, a batch of 512 of 64 x 128 ->
+// 2048 358 for 119.  The chip's clock moves all of the times together, so the
+// choice does not depend on it.  Without a workspace no tile is split.
+namespace {
+
+struct TileCost {
+  int shape, bm, bn, per_cu;
+  double launch, lo, hi, edge, mb_per_us;   // one launch of whole tiles
+  double fixed, split_edge, part_mb_per_us;  // with K ranges: both launches, partial sums
+};
+constexpr TileCost kLarge = {GEMM_MID_NONE, 256, 256, 1, 2.3, 1.08, 1.51, 3.0, 4.5e6, 0, 0, 0};
+constexpr TileCost kMid[2] = {{GEMM_MID_64x128, 64, 128, 2, 1.8, 0.41, 0.68, 3.5, 5.2e6, 4.6, 3.8, 2.4e6},
+                              {GEMM_MID_128x256, 128, 256, 1, 1.1, 0.67, 0.91, 4.5, 5.2e6, 4.5, 5.2, 2.6e6}};
+
+// `units` workgroups in rounds of `slots`, in stage times: lo where one runs
+// alone, hi where the chip is full (the clock falls and the L2s fill).
+double rounds(double units, double slots, const TileCost& c) {
+  const double full = (double)(int64_t)(units / slots), rest = units - full * slots;
+  return full * c.hi + (rest > 0 ? c.lo + (c.hi - c.lo) * rest / slots : 0.0);
+}
+
+// The few-rows kernel: the latency of a wave's passes over K, the work of the
+// workgroups that follow each other on a CU (a workgroup fills it; per
+// projection and 16-row block, and per K chunk for W and each row of X), or
+// the bytes at HBM's rate.
+double rows_cost(double batch, int64_t M, int64_t N, int64_t K, int np, int n_cu, double bytes) {
+  const double mb = (double)((M + 15) / 16), nch = (double)((K + BK - 1) / BK), w = np * mb;
+  const int64_t per_pass = mb <= 2 ? (np == 2 ? 16 : 32) : 16;  // waves x chunks in flight
+  const double passes = (double)(((int64_t)nch + per_pass - 1) / per_pass);
+  const double work = 0.49 + 0.054 * w + nch * (0.066 * np + 0.0033 * (double)M);
+  const double chip = (double)(((int64_t)batch * ((N + 15) / 16) + n_cu - 1) / n_cu) * work;
+  const double latency = passes * 2.3, hbm = bytes / 6.2e6;
+  return 2.15 + (latency > chip ? (latency > hbm ? latency : hbm) : (chip > hbm ? chip : hbm));
+}
+
+GemmMidPlan plan_for(int64_t batch, int64_t M, int64_t N, int64_t K, bool paired, int n_cu, bool ws) {
   GemmMidPlan best{GEMM_MID_NONE, 0, n_cu, 1};
-  const int64_t wrows = paired ? 2 * N : N;
-  // Few rows: gemm_bf16_rows reads W once at HBM rate, but X once per 16
-  // columns.  17 rows: 8.2 against 9.3 us at 2752 -> 1024, 29.7 against 22.9
-  // at 11008 -> 4096; 64 rows, without K ranges: 61 against 89 us.
-  if (gemm_bf16_rows_ok(M, N) && (M <= 16 || (M <= 48 && wrows * K <= 8 << 20) || !ws)) {
+  const int np = paired ? 2 : 1;
+  const double nb = (double)batch, kst = (double)((K + BK - 1) / BK);
+  const double wsize = nb * np * (double)N * (double)K;  // weight elements
+  const double bytes = 2.0 * (wsize + nb * (double)M * (double)(K + N));
+  const bool rows = gemm_bf16_rows_ok(M, N);
+  // At most 16 rows of a long K over many weight bytes: the loads of W bound
+  // every kernel and this one streams them best (8 rows x 4096 -> 131072 193 us
+  // for 212, 1 row x 2048 -> 32768 23 for 33), which the fit underrates.
+  if (rows && M <= 16 && K >= 2048 && wsize >= 1 << 25) {
     best.shape = GEMM_ROWS;
     return best;
   }
-  const double kst = (double)((K + BK - 1) / BK);
-  auto rounds = [&](double units, double slots, double stages, double lo, double hi) {
-    const double full = (double)(int64_t)(units / slots), rest = units - full * slots;
-    return stages * (full * hi + (rest > 0 ? lo + (hi - lo) * rest / slots : 0.0));
+  auto tiles = [&](const TileCost& c) {
+    const int64_t cols = paired ? c.bn / 2 : c.bn;
+    return nb * (double)(((M + c.bm - 1) / c.bm) * ((N + cols - 1) / cols));
   };
-  auto tiles = [&](int bm, int bn) {
-    const int64_t cols = paired ? bn / 2 : bn;
-    return (double)(((M + bm - 1) / bm) * ((N + cols - 1) / cols));
+  auto whole = [&](const TileCost& c) {
+    const double t = (kst + c.edge) * rounds(tiles(c), (double)n_cu * c.per_cu, c), hbm = bytes / c.mb_per_us;
+    return c.launch + (t > hbm ? t : hbm);
   };
-  double cost = rounds(tiles(256, 256), n_cu, kst, 1.05, 1.52) + 4.3;
-  const struct {
-    int shape, bm, bn, per_cu;
-    double lo, hi, launch, reduce, mb_per_us;
-  } shapes[2] = {{GEMM_MID_128x256, 128, 256, 1, 0.63, 0.89, 2.9, 3.8, 3.1},
-                 {GEMM_MID_64x128, 64, 128, 2, 0.27, 0.60, 4.1, 3.0, 2.9}};
-  for (const auto& sh : shapes) {
-    const double t = tiles(sh.bm, sh.bn), slots = (double)n_cu * sh.per_cu;
-    if (!grid_fits((int64_t)t + n_cu, 2 * sh.bn)) continue;  // at most n_cu workgroups for split tiles
-    auto consider = [&](double c, int64_t direct, int64_t splits) {
-      if (c < 0.98 * cost) {
-        cost = c;
-        best = GemmMidPlan{sh.shape, (int)direct, n_cu, (int)splits};
-      }
-    };
-    consider(rounds(t, slots, kst, sh.lo, sh.hi) + sh.launch, (int64_t)t, 1);
+  double cost = whole(kLarge);
+  auto consider = [&](double c, const GemmMidPlan& p) {
+    if (c < cost) {
+      cost = c;
+      best = p;
+    }
+  };
+  // In a batch only where it is clearly cheaper: its fit is the looser one.  A
+  // batch that fills the chip reads its X from memory too, which counts where
+  // that is no smaller than W: 1024 of 64 x 2048 -> 64 257 us for 190.
+  const double margin = batch == 1 ? 1.0 : 1.3;
+  const bool x_counts = batch > 1 && M > 32 && M >= N && K >= 256 && nb * (double)((N + 15) / 16) >= 4.0 * n_cu;
+  if (rows && !x_counts) consider(margin * rows_cost(nb, M, N, K, np, n_cu, bytes), GemmMidPlan{GEMM_ROWS, 0, n_cu, 1});
+  // One row of large tiles on every CU reads W once where two rows of middle
+  // ones read it twice: 256 rows x 512 -> 131072 44 us for 56.
+  if (batch != 1 || (M > 128 && M <= 256 && tiles(kLarge) >= n_cu)) return best;
+  for (const TileCost& c : kMid) {
+    const double t = tiles(c), slots = (double)n_cu * c.per_cu;
+    if (!grid_fits((int64_t)t + n_cu, 2 * c.bn)) continue;  // at most n_cu workgroups for split tiles
+    consider(whole(c), GemmMidPlan{c.shape, (int)t, n_cu, 1});
     if (!ws) continue;
     // K ranges for the tiles past the last whole round, one workgroup per CU
     const int64_t direct = (int64_t)t / n_cu * n_cu, left = (int64_t)t - direct;
-    if (left == 0 || (sh.per_cu > 1 && direct > 0)) continue;
+    if (left == 0 || (c.per_cu > 1 && direct > 0)) continue;
     int64_t splits = n_cu / left;
     if (splits > (int64_t)(kst / 2)) splits = (int64_t)(kst / 2);
     if (splits < 2) continue;
-    consider(rounds((double)direct, slots, kst, sh.lo, sh.hi) +
-                 rounds((double)(left * splits), slots, kst / (double)splits, sh.lo, sh.hi) + sh.launch +
-                 sh.reduce + (double)(left * splits * sh.bm * sh.bn * 4) * 1e-6 / sh.mb_per_us,
-             direct, splits);
+    const double units = (double)(left * splits), hbm = bytes / c.mb_per_us;
+    const double loop = (kst + c.edge) * rounds((double)direct, slots, c) +
+                        (kst / (double)splits + c.split_edge) * rounds(units, slots, c);
+    // only rows below M are written: M of each column of tiles
+    const double part = units * c.bn * 4.0 * (double)M / (double)((M + c.bm - 1) / c.bm);
+    // taken where it is clearly cheaper, and for calls that the host's two
+    // launches and the workspace (13 us) do not bound anyway: 128 rows x 1024
+    // -> 1024 13.2 us for 8.4 whole
+    const double t2 = 1.05 * (c.fixed + (loop > hbm ? loop : hbm) + part / c.part_mb_per_us);
+    consider(t2 > 13.0 ? t2 : 13.0, GemmMidPlan{c.shape, (int)direct, n_cu, (int)splits});
   }
   return best;
 }
 
-GemmMidPlan gemm_bf16_plan(int64_t batch, int64_t M, int64_t N, int64_t K, bool paired, int n_cu, int64_t ws_bytes) {
-  if (batch != 1) return GemmMidPlan{gemm_bf16_rows_ok(M, N) ? GEMM_ROWS : GEMM_MID_NONE, 0, n_cu, 1};
-  if (ws_bytes > 0) {
-    const GemmMidPlan p = gemm_bf16_mid_plan(M, N, K, paired, n_cu, true);
-    if (gemm_bf16_mid_workspace(p, M, N, paired) <= ws_bytes) return p;
-  }
-  return gemm_bf16_mid_plan(M, N, K, paired, n_cu, false);
-}
+}  // namespace
 
 int64_t gemm_bf16_mid_workspace(const GemmMidPlan& p, int64_t M, int64_t N, bool paired) {
   if (p.shape < GEMM_MID_128x256 || p.splits <= 1) return 0;
@@ -361,6 +400,14 @@ int64_t gemm_bf16_mid_workspace(const GemmMidPlan& p, int64_t M, int64_t N, bool
   const int64_t cols = paired ? bn / 2 : bn;
   const int64_t left = ((M + bm - 1) / bm) * ((N + cols - 1) / cols) - p.direct;
   return left * p.splits * bm * bn * (int64_t)sizeof(float);
+}
+
+GemmMidPlan gemm_bf16_plan(int64_t batch, int64_t M, int64_t N, int64_t K, bool paired, int n_cu, int64_t ws_bytes) {
+  if (batch == 1 && ws_bytes > 0) {
+    const GemmMidPlan p = plan_for(1, M, N, K, paired, n_cu, true);
+    if (gemm_bf16_mid_workspace(p, M, N, paired) <= ws_bytes) return p;
+  }
+  return plan_for(batch, M, N, K, paired, n_cu, false);
 }
 
 int32_t gemm_bf16_mid_launch(const GemmMidPlan& plan, int32_t epi, int64_t M, int64_t N, int64_t K, const void* x,

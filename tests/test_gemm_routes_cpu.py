@@ -31,6 +31,29 @@ def test_bf16_grids_stay_within_a_launch(M, N, epi, batch):
     assert groups * threads < 1 << 32
 
 
+# Products that some other kernel runs at least 1.4 times as fast as the
+# few-rows kernel or (the last three) the middle tiles do.
+@pytest.mark.parametrize("M,N,K,epi,batch,routes", [
+    (64, 131072, 4096, L.EPI_NONE, 1, {M128, M64, LARGE}), (33, 131072, 512, L.EPI_NONE, 1, {M128, M64, LARGE}),
+    (16, 131072, 512, L.EPI_NONE, 1, {M128, M64, LARGE}), (64, 65536, 4096, L.EPI_SILU_MUL, 1, {M128, M64, LARGE}),
+    (64, 2048, 128, L.EPI_NONE, 512, {LARGE}), (17, 1024, 1024, L.EPI_NONE, 256, {LARGE}),
+    (64, 4096, 4096, L.EPI_NONE, 32, {LARGE}), (256, 131072, 64, L.EPI_NONE, 1, {LARGE}),
+    (200, 131072, 512, L.EPI_NONE, 1, {LARGE}), (1000, 65536, 64, L.EPI_NONE, 1, {LARGE})])
+def test_bf16_few_rows_and_short_k(M, N, K, epi, batch, routes):
+    for ws in (0, 1 << 40):
+        assert route(BF16, M, N, K, epi, batch, ws)[0] in routes
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 40, 64, 65, 200, 333, 1000, 3000])
+@pytest.mark.parametrize("N,K", [(256, 4096), (1024, 1024), (4096, 11008), (131072, 64), (65536, 4096)])
+@pytest.mark.parametrize("epi", [L.EPI_NONE, L.EPI_SILU_MUL])
+def test_no_workspace_is_the_plan_of_a_call_that_asks_for_none(M, N, K, epi):
+    """A plan that splits no tile asks for no workspace: the launch that follows has none and must plan the same."""
+    r, plan = route(BF16, M, N, K, epi)
+    if plan[1] == 0:
+        assert route(BF16, M, N, K, epi, ws=0) == (r, plan)
+
+
 def test_f32_grids_stay_within_a_launch():
     # 2 x 2^23 tiles of 256 work-items: the general kernel, with a grid of two dimensions
     assert route(F32, 65, 1 << 29, 4)[0] == GENERAL
