@@ -49,6 +49,7 @@ SIGNATURES: dict[str, tuple] = {
         [_i32, _i64, _i64, _i64, _i64, _i64, _i64, _p, _pi64, _p, _pi64, _p, _pi64,
          _f32, _i32, _i64, _p, _i64, _i32, _p, _pi64, _p, _p, _p],
     ),
+    "catopt_hip_attn_route": (_i32, [_i64, _i64, _i64, _i64, _i64, _i32]),
     "catopt_hip_attn_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64]),
     "catopt_hip_attn_fwd_ws": (
         _i32,

@@ -729,6 +729,33 @@ bool q64_pays(int64_t heads, int64_t Tq, int* paired) {
   return wgs * 100 >= slots * (slots == kCus ? 70 : 85);
 }
 
+// Whether the few-query kernel (Tq <= kAttnSplitQueries) pays for `heads` heads
+// of Tq queries and Tk keys.  What it gains is ranges of keys in parallel and
+// whole-stage loads; a workgroup of it holds 64 KB of LDS for its stage pair,
+// where five of the 32-query kernel's at d = 64 share a CU, and walks 32 keys
+// a wave, which takes more instructions per score.  So the 32-query kernel
+// keeps, in us, few-query / 32-query:
+//   d = 64, over 2048 heads, half a key stage: 4096 x 64 keys 26 / 20 (1
+//   query) and 30 / 21 (32); with more than 16 queries a whole one, 34 / 32;
+//   and with a plane a half-filled second round of 512, 768 x 512 52 / 46;
+//   d = 128, two key ranges (their combine costs what they give), more than
+//   16 queries: 256 heads x 1000 keys 30 / 25;
+//   d = 128 unsplit: from 1024 heads, more than 16 queries and at most 128
+//   keys, 2048 x 100 33 / 29; with a mask or bias plane from 512 heads and
+//   more than 8 queries, 2048 x 250 94 / 77.
+bool few_pays(int64_t heads, int64_t Tq, int64_t Tk, int64_t d, int32_t mode) {
+  const bool plane = mode == CATOPT_MASK_BOOL || mode == CATOPT_MASK_BIAS;
+  if (d == 64) {
+    if (plane && Tq > 16 && heads > 512 && heads < 1024) return false;
+    return heads <= 2048 || Tk > (Tq > 16 ? 128 : 64);
+  }
+  const int64_t n = attn_split_count(heads, 1, Tk, d);
+  if (n == 2) return Tq <= 16;
+  if (n > 2) return true;
+  if (plane && heads >= 512) return Tq <= 8;
+  return heads < 1024 || Tq <= 16 || Tk > 128;
+}
+
 template <int D, int MASK>
 int32_t attn_launch(const uint16_t* q, const int64_t* qs, const uint16_t* k, const int64_t* ks,
                     const uint16_t* v, const int64_t* vs, uint16_t* o, const int64_t* os,
@@ -784,7 +811,18 @@ using namespace catopt;
 extern "C" int64_t catopt_hip_attn_workspace_bytes(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t d) {
   if (B < 0 || H < 0 || Tq < 0 || Tk < 0 || (d != 64 && d != 128)) return -1;
   if (B == 0 || H == 0 || Tq == 0 || Tq > kAttnSplitQueries || B > 65535 || H > 65535 || Tk > 0x7fffffffLL) return 0;
-  return attn_split_workspace(B, H, Tq, Tk, d);
+  // where keys are split, the choice of kernel does not depend on the mask mode
+  return few_pays(B * H, Tq, Tk, d, CATOPT_MASK_NONE) ? attn_split_workspace(B, H, Tq, Tk, d) : 0;
+}
+
+extern "C" int32_t catopt_hip_attn_route(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t d, int32_t mask_mode) {
+  if (B < 1 || H < 1 || Tq < 1 || Tk < 0 || (d != 64 && d != 128)) return -1;
+  if (mask_mode < CATOPT_MASK_NONE || mask_mode > CATOPT_MASK_BIAS) return -1;
+  if (Tq <= kAttnSplitQueries && few_pays(B * H, Tq, Tk, d, mask_mode)) return CATOPT_ATTN_FEW_QUERIES;
+  const int64_t st[3] = {H * Tk * d, Tk * d, d};
+  int paired = 0;
+  if (!q64_fits(d, mask_mode, Tk, st, st) || !q64_pays(B * H, Tq, &paired)) return CATOPT_ATTN_32_QUERIES;
+  return paired ? CATOPT_ATTN_64_QUERIES_PAIRED : CATOPT_ATTN_64_QUERIES;
 }
 
 extern "C" int32_t catopt_hip_attn_fwd_ws(int32_t dtype, int64_t B, int64_t H, int64_t Tq,
@@ -821,7 +859,7 @@ extern "C" int32_t catopt_hip_attn_fwd_ws(int32_t dtype, int64_t B, int64_t H, i
   auto kp = static_cast<const uint16_t*>(k);
   auto vp = static_cast<const uint16_t*>(v);
   auto op = static_cast<uint16_t*>(o);
-  if (Tq <= kAttnSplitQueries) {
+  if (Tq <= kAttnSplitQueries && few_pays(B * H, Tq, Tk, d, mask_mode)) {
     AttnArgs a{qp, kp, vp, op, {}, {}, {}, {}, m_out, l_out, B, H, Tq, Tk, causal_off, mask, mask_ld, scale, normalize};
     for (int i = 0; i < 3; ++i) {
       a.qs[i] = q_strides[i];

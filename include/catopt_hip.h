@@ -207,7 +207,7 @@ int32_t catopt_hip_attn_fwd(int32_t dtype, int64_t B, int64_t H, int64_t Tq,
 
 /*
  * catopt_hip_attn_fwd with a workspace: a call with few queries (Tq <= 32)
- * then splits the keys of each (b, h) over workgroups and combines the
+ * and few heads then splits the keys of each (b, h) over workgroups and combines the
  * ranges' carriers (the workspace holds them).
  * catopt_hip_attn_workspace_bytes is the size such a call reads (0: none,
  * -1: invalid arguments); with less, or NULL, the keys are not split.
@@ -223,7 +223,21 @@ int32_t catopt_hip_attn_fwd_ws(int32_t dtype, int64_t B, int64_t H, int64_t Tq,
                             int64_t mask_ld, int32_t normalize, void* o,
                             const int64_t* o_strides, float* m_out,
                             float* l_out, void* workspace,
-                               int64_t workspace_bytes, void* stream);
+                            int64_t workspace_bytes, void* stream);
+
+/*
+ * The kernel a catopt_hip_attn_fwd_ws call with contiguous heads runs on (a
+ * catopt_attn_route, or -1 for invalid arguments), for tests and tools: host
+ * only, no device needed.
+ */
+enum catopt_attn_route {
+  CATOPT_ATTN_32_QUERIES = 0,        /* 32 queries per wave, any mask */
+  CATOPT_ATTN_64_QUERIES = 1,        /* d = 128, whole key tiles, no plane: 64 per wave */
+  CATOPT_ATTN_64_QUERIES_PAIRED = 2, /* the same, two query tiles per workgroup */
+  CATOPT_ATTN_FEW_QUERIES = 3        /* Tq <= 32: keys over workgroups and waves */
+};
+int32_t catopt_hip_attn_route(int64_t B, int64_t H, int64_t Tq, int64_t Tk,
+                              int64_t d, int32_t mask_mode);
 
 /*
  * Row statistics of an explicit score block for the om element
