@@ -248,7 +248,7 @@ using namespace catopt;
 extern "C" int64_t catopt_hip_linear_workspace_bytes(int32_t dtype, int64_t M, int64_t N, int64_t K,
                                                      int32_t epilogue) {
   if (M < 0 || N < 0 || K < 0 || epilogue < CATOPT_EPI_NONE || epilogue > CATOPT_EPI_GLU) return -1;
-  if (dtype != CATOPT_BF16 || M == 0 || N == 0 || K == 0) return 0;
+  if (dtype != CATOPT_BF16 || M == 0 || N == 0 || K == 0 || K % 8) return 0;  // K % 8: the general kernel
   if (M > 0x7fffffffLL || N > 0x3fffffffLL || K > 0x7fffffffLL) return 0;
   int n_cu = 0;
   if (gemm_cu_count(&n_cu) != CATOPT_OK) return 0;  // no device: nothing will be launched

@@ -106,6 +106,11 @@ def test_linear_without_workspace_and_with_too_little(epi):
         _check(y, *ref)
 
 
+def test_no_workspace_for_the_general_kernel():
+    q = L.load().catopt_hip_linear_workspace_bytes
+    assert q(L.BF16, 100, 512, 4096, L.EPI_NONE) > 0 and q(L.BF16, 100, 512, 4097, L.EPI_NONE) == 0
+
+
 @pytest.mark.parametrize("nb,M,N,Kd", [(3, 1, 40, 64), (5, 20, 96, 136), (2, 64, 33, 256)])
 def test_batched_few_rows(nb, M, N, Kd):
     g = torch.Generator(device=DEV).manual_seed(nb + M)
