@@ -60,7 +60,8 @@ def _check(q, k, v, scale, **kw):
 
 
 SHAPES = [(1, 1, 1, 1), (1, 2, 1, 33), (2, 3, 5, 64), (1, 5, 32, 127), (1, 4, 7, 128), (2, 12, 1, 1000), (1, 1, 2, 4096),
-          (3, 40, 1, 700), (1, 600, 3, 130), (1, 8, 31, 2049)]
+          (3, 40, 1, 700), (1, 600, 3, 130), (1, 8, 31, 2049),
+          (1, 4, 33, 700)]  # one query past the kernel
 
 
 @pytest.mark.parametrize("d", [64, 128, 40])
@@ -73,7 +74,7 @@ def test_unmasked_and_causal(B, H, Tq, Tk, d):
 
 
 @pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("Tq,Tk", [(1, 63), (6, 513), (32, 3000)])
+@pytest.mark.parametrize("Tq,Tk", [(1, 63), (6, 513), (32, 3000), (33, 513)])
 def test_planes(Tq, Tk, d):
     q, k, v = _case(2, 3, Tq, Tk, d, seed=Tk)
     g = torch.Generator(device=DEV).manual_seed(1)

@@ -70,9 +70,11 @@ def _release():
 # ------------------------------------------------------------- GEMM grids
 
 
-# M = 2304: 9 M-tiles of 256, so the tile order has one full group of 8
-# M-tiles and a partial last group of 1; N = 2048 (or 1024 paired outputs):
-# 8 N-tiles, 72 workgroups, a multiple of 8, so the XCD remap runs.
+# M = 2304, N = 2048 (or 1024 paired outputs): the 128 x 256 tiles, 18 M-tiles
+# in two full groups of 8 and a part of one, 144 workgroups, a multiple of 8.
+# (The persistent 256 x 256 tiles' ragged sizes and epilogues are in
+# test_gemm_bf16_sizes_gpu.py; here test_linear_persistent_rounds_ragged and
+# the C2 shapes run them.)
 @pytest.mark.parametrize("epi", [L.EPI_NONE, L.EPI_BIAS, L.EPI_BIAS_ADD2])
 def test_linear_grouped_grid(dev, epi):
     M, N, Kd = 2304, 2048, 512
@@ -100,8 +102,8 @@ def test_linear_paired_grouped_grid(dev, epi):
 
 
 def test_linear_large_plain(dev):
-    # M·N·K = 2^30, 16 tiles: the plain (no-epilogue) GEMM of the down
-    # projection's kind on a grid whose workgroups take one tile each
+    # M·N·K = 2^30: the plain (no-epilogue) GEMM of the down projection's kind
+    # on the 64 x 128 tiles, one to a workgroup
     M = N = Kd = 1024
     x = _rand((M, Kd), torch.bfloat16, 47)
     w = _rand((N, Kd), torch.bfloat16, 48, 0.05)
@@ -142,10 +144,9 @@ def test_linear_persistent_rounds_ragged(dev, epi):
 
 
 # Grids that are multiples of 8 workgroups, so the XCD remaps and (causal)
-# the tile orders run: d = 128, T = 256 is the 64-query kernel with one
-# query tile per workgroup (8 workgroups), T = 512 the same kernel with the
-# two tiles of a head's pair per workgroup (8 workgroups, 8 heads: one per
-# XCD), and d = 64 the 32-query kernel (B·H·⌈T/128⌉ = 16 workgroups).
+# the tile orders run, on the 32-query kernel (so few tiles leave the 64-query
+# kernel's CUs idle): B·H·⌈T/128⌉ = 16 or 32 workgroups at d = 128, 16 at d = 64.
+# The 64-query kernel's grids are in test_attn_routes_gpu.py.
 @pytest.mark.parametrize("T,d", [(256, 128), (512, 128), (256, 64)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_attention_remapped_grid(dev, causal, T, d):

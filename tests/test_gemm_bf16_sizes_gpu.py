@@ -22,6 +22,16 @@ DEV = "cuda:0"
 BF = torch.bfloat16
 
 
+ROWS, M128, M64, LARGE = 1, 2, 3, 4  # catopt_gemm_route
+
+
+def _route(M, N, Kd, epi, batch=1):
+    """(route, tiles done whole, tiles split, K ranges) on this device, with a workspace."""
+    plan = L.i64_array([0, 0, 0])
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return (L.load().catopt_hip_gemm_route(L.BF16, batch, M, N, Kd, epi, cus, 1 << 40, plan), *plan)
+
+
 def _rows(g, r, k, pad):
     """(r, k) bf16 rows of stride k + pad, the padding full of Inf and NaN."""
     t = torch.full((r, k + pad), float("inf"), dtype=BF, device=DEV)
@@ -73,7 +83,7 @@ def test_linear_sizes(M, N, Kd, epi, pad):
 
 
 # the middle tiles: one row past the few-row kernels, tile edges either side,
-# whole tiles only, K ranges (with a K tail), a last round split in ranges, odd N
+# whole tiles only, every tile's K in ranges (with a K tail), odd N
 MID = [(65, 256, 4096), (64, 1024, 4104), (128, 4096, 1032), (129, 130, 2056), (200, 1003, 2048), (333, 640, 5000),
        (257, 4096, 520), (400, 11008, 72), (1000, 2752, 264), (300, 11010, 1024)]
 
@@ -81,6 +91,35 @@ MID = [(65, 256, 4096), (64, 1024, 4104), (128, 4096, 1032), (129, 130, 2056), (
 @pytest.mark.parametrize("epi", [L.EPI_NONE, L.EPI_BIAS, L.EPI_BIAS_ADD2, L.EPI_SILU_MUL, L.EPI_GLU])
 @pytest.mark.parametrize("M,N,Kd", MID)
 def test_linear_middle_sizes(M, N, Kd, epi):
+    test_linear_sizes(M, N, Kd, epi, 16 if M % 2 else 0)
+
+
+# Whole rounds of tiles and K ranges for those left over, ragged M and N and K
+# tails: one and two whole rounds, 2 to 83 tiles split into 2 to 32 ranges.
+MIXED = [(333, 11008, 4096, L.EPI_SILU_MUL), (300, 11008, 2056, L.EPI_GLU), (395, 8456, 4104, L.EPI_SILU_MUL),
+         (700, 11008, 4104, L.EPI_NONE), (700, 11003, 2056, L.EPI_BIAS_ADD2), (1000, 8456, 4104, L.EPI_GLU),
+         (1500, 11008, 2056, L.EPI_BIAS), (2050, 4355, 4104, L.EPI_SILU_MUL)]
+
+
+@pytest.mark.parametrize("M,N,Kd,epi", MIXED)
+def test_linear_whole_rounds_and_split_tiles(M, N, Kd, epi):
+    route, whole, split, ranges = _route(M, N, Kd, epi)
+    assert route in (M128, M64) and whole > 0 and split > 0 and ranges > 1
+    test_linear_sizes(M, N, Kd, epi, 0)
+
+
+# The persistent 256 x 256 tiles: one row of tiles and ten (a whole group of
+# eight and a part of one), one to three rounds, ragged M, N and K, stores of
+# whole rows (N a multiple of 8) and column by column.
+LARGE_SIZES = [(250, 65541, 264), (1003, 33000, 72), (2310, 8201, 72), (2310, 16400, 136), (4160, 8200, 1032)]
+
+
+@pytest.mark.parametrize("epi", [L.EPI_NONE, L.EPI_BIAS, L.EPI_BIAS_ADD2, L.EPI_SILU_MUL, L.EPI_GLU])
+@pytest.mark.parametrize("M,N,Kd", LARGE_SIZES)
+def test_linear_large_tiles(M, N, Kd, epi):
+    if epi in (L.EPI_SILU_MUL, L.EPI_GLU):
+        N = N // 2
+    assert _route(M, N, Kd, epi)[0] == LARGE
     test_linear_sizes(M, N, Kd, epi, 16 if M % 2 else 0)
 
 
@@ -111,8 +150,13 @@ def test_no_workspace_for_the_general_kernel():
     assert q(L.BF16, 100, 512, 4096, L.EPI_NONE) > 0 and q(L.BF16, 100, 512, 4097, L.EPI_NONE) == 0
 
 
-@pytest.mark.parametrize("nb,M,N,Kd", [(3, 1, 40, 64), (5, 20, 96, 136), (2, 64, 33, 256)])
-def test_batched_few_rows(nb, M, N, Kd):
+# few rows, and batches that the large tiles run: few rows over many workgroups,
+# rows past the few-row kernels (ragged, a K tail, C rows not 16-byte aligned)
+@pytest.mark.parametrize("nb,M,N,Kd,route", [(3, 1, 40, 64, ROWS), (5, 20, 96, 136, ROWS), (2, 64, 33, 256, ROWS),
+                                             (200, 33, 1030, 136, LARGE), (40, 64, 4096, 72, LARGE),
+                                             (3, 70, 300, 264, LARGE), (2, 513, 259, 72, LARGE)])
+def test_batched_products(nb, M, N, Kd, route):
+    assert _route(M, N, Kd, L.EPI_NONE, nb)[0] == route
     g = torch.Generator(device=DEV).manual_seed(nb + M)
     a = torch.randn((nb, M, Kd), generator=g, device=DEV).to(BF)
     b = torch.randn((nb, N, Kd), generator=g, device=DEV).to(BF)

@@ -227,12 +227,12 @@ def test_attention_causal_offset_and_cross_lengths(dev):
     _gate(ref, o, TOL_BF16)
 
 
-# The 64-query kernel (attn_q64_kernel) takes d = 128, no mask or causal, and
-# whole 64-key tiles; these cases reach its edges: query counts off a
-# multiple of the 256-query workgroup and of a wave's 64, keys of one and of
-# many tiles, causal offsets that start, end or empty rows, several heads per
-# XCD and a head count off a multiple of 8 (the grid mappings), and odd and
-# even query-tile counts (even counts run two tiles per workgroup).
+# d = 128, no mask or causal, and whole 64-key tiles, which the 64-query kernel
+# takes too where its workgroups fill the chip (test_attn_routes_gpu.py); these
+# few heads run on the 32-query kernel.  Query counts off a multiple of a
+# workgroup's and of a wave's, keys of one and of many tiles, causal offsets
+# that start, end or empty rows, several heads per XCD and a head count off a
+# multiple of 8 (the grid mappings).
 @pytest.mark.parametrize("B,H,Tq,Tk,causal,off", [
     (1, 2, 256, 256, True, 0), (2, 3, 100, 320, True, 220), (1, 16, 300, 512, True, 0),
     (1, 2, 200, 64, False, 0), (1, 4, 512, 512, True, -130), (1, 2, 64, 1024, True, 960),
@@ -274,7 +274,6 @@ def test_attention_q64_strided_and_zero_rows(dev):
     assert bool((o[:, :, :40] == 0).all())
 
 
-# one query tile per workgroup (192 queries) and two (448: the paired path)
 @pytest.mark.parametrize("Tq,Tk,causal", [(192, 256, False), (448, 512, True)])
 def test_attention_q64_unnormalised_numerator(dev, Tq, Tk, causal):
     q, k, v = _qkv(1, 2, Tq, 128, 450, Tk=Tk)
