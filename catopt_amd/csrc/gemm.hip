@@ -1,10 +1,10 @@
 // GEMM entry points: catopt_hip_linear and catopt_hip_matmul.
 //
 // bf16 with K-contiguous, 16-byte aligned operands goes to the bf16 MFMA
-// kernels (gemm_bf16.hip, gemm_bf16_mid.hip, gemm_bf16_skinny.hip by size).  Everything else — fp32 (the weight
-// chain of the linear-bias association form and its construction-time
-// fold), transposed operands, unaligned views — runs here on a 64x64-tile
-// kernel using the 32x32x2 fp32 MFMA, with operands staged through LDS in
+// kernels (gemm_bf16.hip, gemm_bf16_mid.hip, gemm_bf16_skinny.hip by size),
+// fp32 with few rows to the kernel below, other aligned fp32 to
+// gemm_f32_tile.hip.  Everything else — K-strided or unaligned bf16, unaligned
+// fp32, paired fp32 epilogues — runs here on a 64x64-tile kernel using the 32x32x2 fp32 MFMA, with operands staged through LDS in
 // k-contiguous order whatever their global layout.  bf16 operands are
 // widened to fp32 in LDS (the products are exact), so both paths
 // accumulate in fp32.

@@ -14,7 +14,7 @@
 // 64 through a ring of STAGES LDS slots: both operands' rows go global->LDS
 // directly (whole 128-byte lines, rows XOR-swizzled so that a fragment read
 // hits 16 distinct 16-byte bank groups), STAGES - 1 stages ahead, with one
-// barrier per stage.  What bounds the loop is the stage's load latency and
+// barrier per stage.  What bounds the loop is the stage's loads, by latency or
 // bytes: 0.63 us per 128 x 256 x 64 stage with the operands cached, 0.80 us
 // with W from HBM, where the MFMAs take 0.4 us.  A two-slot ring of 128 x 128
 // tiles, two workgroups per CU, needed 0.83 us for the same work and cached

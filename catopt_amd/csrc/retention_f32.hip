@@ -20,7 +20,7 @@
 // at d = 128.  (With a workgroup per 32 value columns and all of a head's
 // chunks in order, each slice recomputed the scores and each wave the whole
 // P v.)  Measured, that kernel and this one: 32 heads x 2048 steps x 128
-// 253 / 103 us, 64 x 8192 x 128 1011 / 600, 32 x 2048 x 64 221 / 45.  A product
+// 255 / 96 us, 64 x 8192 x 128 1009 / 588, 32 x 2048 x 64 219 / 45.  A product
 // takes 38-40 ns here (27 at 2.4 GHz; without the loads the 64 x 8192 output
 // pass still takes 409 of 471 us).  With MFMA accumulators in VGPRs
 // (-amdgpu-mfma-vgpr-form) d = 128 is 5% faster and d = 64 16-25% slower: two

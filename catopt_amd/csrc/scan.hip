@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kThreads) void affd_chunk_apply(
 // Thread layout: TPD = N/4 threads per channel d, each owning 4 consecutive
 // state elements n (one 16-byte load of a per step); DPW = 256/TPD channels
 // per workgroup; grid.y = batch.  y[b,t,d] is reduced across the TPD lanes
-// of a channel with xor shuffles (DPP quad-perm / ds_swizzle patterns).
+// of a channel with DPP moves.
 template <int N>
 struct SsmLayout {
   static constexpr int TPD = N / 4;
