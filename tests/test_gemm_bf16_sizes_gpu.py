@@ -150,12 +150,8 @@ def test_no_workspace_for_the_general_kernel():
     assert q(L.BF16, 100, 512, 4096, L.EPI_NONE) > 0 and q(L.BF16, 100, 512, 4097, L.EPI_NONE) == 0
 
 
-# few rows, and batches that the large tiles run: few rows over many workgroups,
-# rows past the few-row kernels (ragged, a K tail, C rows not 16-byte aligned)
-@pytest.mark.parametrize("nb,M,N,Kd,route", [(3, 1, 40, 64, ROWS), (5, 20, 96, 136, ROWS), (2, 64, 33, 256, ROWS),
-                                             (200, 33, 1030, 136, LARGE), (40, 64, 4096, 72, LARGE),
-                                             (3, 70, 300, 264, LARGE), (2, 513, 259, 72, LARGE)])
-def test_batched_products(nb, M, N, Kd, route):
+@pytest.mark.parametrize("nb,M,N,Kd", [(3, 1, 40, 64), (5, 20, 96, 136), (2, 64, 33, 256)])
+def test_batched_few_rows(nb, M, N, Kd, route=ROWS):
     assert _route(M, N, Kd, L.EPI_NONE, nb)[0] == route
     g = torch.Generator(device=DEV).manual_seed(nb + M)
     a = torch.randn((nb, M, Kd), generator=g, device=DEV).to(BF)
@@ -163,6 +159,13 @@ def test_batched_products(nb, M, N, Kd, route):
     y = K.matmul(a, b.transpose(-1, -2))
     for i in range(nb):
         _check(y[i], *_reference(a[i], b[i], L.EPI_NONE, None, None))
+
+
+# batches that the large tiles run: few rows over many workgroups, rows past the
+# few-row kernel (ragged, a K tail, C rows not 16-byte aligned)
+@pytest.mark.parametrize("nb,M,N,Kd", [(200, 33, 1030, 136), (40, 64, 4096, 72), (3, 70, 300, 264), (2, 513, 259, 72)])
+def test_batched_large_tiles(nb, M, N, Kd):
+    test_batched_few_rows(nb, M, N, Kd, LARGE)
 
 
 def test_linear_more_weight_rows_than_the_few_row_grid_takes():
